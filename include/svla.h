@@ -206,10 +206,18 @@ int svla_slab_block_bf16(const void* x, int ldx, void* out, int rows, int k, svl
 #define SVLA_TILE_STRICT 0x100
 int svla_gemm_set_tile(int tile);
 
-/* Query: the tile configuration (numbering of svla_gemm_set_tile) that
+/* Query: the tile configuration (numbering of svla_gemm_set_tile) among the
+ * forceable ones that
  * svla_linear_bf16 picks for a dense, un-normalised, packed (ldc = n) problem
  * of this shape, or SVLA_EINVAL.  For reports and tests. */
 int svla_gemm_tile_choice(int m, int n, int k, int act);
+
+/* Query: the block tile (rows * 1000 + columns) of the K-split line-DMA kernel
+ * (csrc/gemm_stream.hip) that an automatic call with dense, well aligned
+ * operands and no fused norm runs on -- plain epilogue, or `paired` (RoPE /
+ * SiLU) -- or 0 where it runs on the configuration svla_gemm_tile_choice
+ * names.  These kernels are not among the forceable configurations. */
+int svla_gemm_stream_choice(int m, int n, int k, int paired);
 
 /* Tuning hook: force the number of cross-workgroup K splits of skinny
  * (M <= 256) GEMMs, 1..64 (1 = never split), or -1 for the automatic choice

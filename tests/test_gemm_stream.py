@@ -1,0 +1,139 @@
+"""The K-split line-DMA GEMMs (csrc/gemm_stream.hip): which tile an automatic
+call takes (host-only query) and every tile against an fp32 product, at ragged
+rows, columns and K.
+
+Bound: the kernels accumulate bf16 products in fp32 (K <= 3072 terms: relative
+error below K * 2^-24 < 2e-4 of the sum of magnitudes, far under a bf16 ulp)
+and round once per rounding point, so an output is at most one bf16 ulp
+(2^-7 relative at a binade's edge) from the fp32 reference rounded the same
+way, plus an absolute floor of the accumulation error at outputs near zero."""
+
+import math
+
+import pytest
+import torch
+
+BF16 = torch.bfloat16
+
+# (m, n, k, paired) -> tile: every configuration, on shapes the engine and the
+# layers run and on ragged ones
+CHOICES = [
+    (1600, 720, 960, 0, 64080),      # batch-32 expert O
+    (1600, 1600, 720, 1, 64160),     # batch-32 expert QKV
+    (1600, 4096, 720, 1, 256128),    # batch-32 expert gate|up
+    (7712, 960, 2560, 0, 256128),    # batch-32 prefix down
+    (1665, 960, 2560, 0, 128064),    # five prompts of 333: down
+    (1024, 768, 768, 0, 64064),      # one image: O
+    (1024, 3072, 768, 0, 128096),    # one image: up
+    (5103, 768, 3072, 0, 128128),    # seven images of 729 tokens: down
+    (5103, 2304, 768, 0, 128192),    # seven images of 729 tokens: QKV
+    (2723, 1600, 720, 1, 192128),    # an odd batch: QKV
+    (1999, 768, 3000, 0, 64096),
+    (241, 960, 960, 0, 0),           # batch-1 prefix: the 32-row small tiles
+    (50, 4096, 720, 1, 0),           # batch-1 expert layer: the skinny tile
+    (98304, 3072, 768, 0, 0),        # batch-32 ViT: the 256x256 kernel
+    (300, 64, 56, 0, 0),             # under one K stage
+]
+
+
+@pytest.mark.parametrize("m,n,k,paired,tile", CHOICES)
+def test_choice(m, n, k, paired, tile):
+    from smolvla import _lib
+    assert _lib.load().svla_gemm_stream_choice(m, n, k, paired) == tile
+
+
+def test_choice_refuses_what_the_gemm_refuses():
+    from smolvla import _lib
+    for bad in ((0, 64, 64, 0), (8, 60, 64, 0), (8, 64, 60, 0), (8, 96, 64, 1), (8, 64, 0, 0)):
+        assert _lib.load().svla_gemm_stream_choice(*bad) == -22
+
+
+def _close(got, want, *through):
+    """``through``: the rounded intermediates; one that rounds the other way
+    (its fp32 sum taken in another order) moves the output by its own ulp."""
+    got, want = got.float().cpu(), want.float()
+    tol = 2e-3 * want.abs().mean()
+    for t in (want, *through):
+        tol = tol + 2 ** -7 * t.abs()
+    bad = (got - want).abs() > tol
+    assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} off, " \
+                          f"max {(got - want).abs().max().item():.3e}"
+
+
+# one shape per tile (rows and columns off the tile, K off the 64-deep stage),
+# and the smallest problem: one tile, one stage
+RAGGED = [(1601, 728, 968), (1590, 1608, 712), (1601, 4104, 720), (1665, 968, 2552),
+          (1021, 776, 776), (1021, 3064, 760), (5103, 776, 3064), (5100, 2312, 776),
+          (2723, 1608, 712), (1999, 776, 3000), (520, 64, 64), (513, 24, 72)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", RAGGED)
+def test_plain_epilogues(m, n, k):
+    """bias, scale, GELU / SiLU and an in-place residual; A and W are strided
+    views whose padding is NaN (nothing past K may be read into a product)."""
+    from smolvla import _lib, ops
+    assert _lib.load().svla_gemm_stream_choice(m, n, k, 0) > 0
+    g = torch.Generator().manual_seed(m + n + k)
+    ld = (k + 63) // 64 * 64 + 8
+    a = torch.full((m, ld), float("nan"), dtype=BF16)
+    w = torch.full((n, ld), float("nan"), dtype=BF16)
+    a[:, :k] = torch.randn(m, k, generator=g).to(BF16)
+    w[:, :k] = (torch.randn(n, k, generator=g) * 0.05).to(BF16)
+    b = (torch.randn(n, generator=g) * 0.5).to(BF16)
+    r = torch.randn(m, n, generator=g).to(BF16)
+    A, W, B = a.cuda()[:, :k], w.cuda()[:, :k], b.cuda()
+    y = (a[:, :k].float() @ w[:, :k].float().t())
+    _close(ops.linear(A, W, bias=B, alpha=0.5), (0.5 * y + b.float()).to(BF16))
+    h = (y + b.float()).to(BF16).float()
+    _close(ops.linear(A, W, bias=B, act="gelu_tanh"),
+           torch.nn.functional.gelu(h, approximate="tanh").to(BF16), h)
+    _close(ops.linear(A, W, bias_f32=B.float(), act="silu"),
+           torch.nn.functional.silu(h).to(BF16), h)
+    x = r.cuda()
+    ops.linear(A, W, bias=B, res=x, out=x)
+    _close(x, (h + r.float()).to(BF16), h)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1590, 1600, 712), (1601, 960, 720), (1601, 4096, 720),
+                                   (2723, 1600, 720), (1665, 1600, 968), (513, 1600, 72),
+                                   (700, 5120, 960)])
+def test_paired_epilogues(m, n, k):
+    """RoPE (with remainders; V columns as projected, their remainders
+    untouched) and SiLU(gate) * up, tiles that start inside a 64-column pair
+    block included."""
+    from smolvla import _lib, ops
+    assert _lib.load().svla_gemm_stream_choice(m, n, k, 1) > 0
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(BF16)
+    w = (torch.randn(k, n, generator=g) * 0.05).to(BF16)
+    proj = (a.float() @ w.float()).to(BF16).float()
+    L, rot = 37, n - 320
+    cos_t, sin_t = ops.rope_table(L, 64, 1e5)
+    lo = torch.full((m, n), 7.0, dtype=BF16, device="cuda")
+    hi = ops.linear_rope(a.cuda(), ops.pack_weight(w.cuda()), rot, L, cos_t, sin_t, out_lo=lo)
+    pos = torch.arange(m) % L
+    c, s = cos_t.cpu()[pos][:, None], sin_t.cpu()[pos][:, None]
+    x = proj.view(m, n // 64, 64)
+    want = torch.cat([x[..., :32] * c - x[..., 32:] * s, x[..., 32:] * c + x[..., :32] * s],
+                     -1).reshape(m, n)
+    want[:, rot:] = proj[:, rot:]
+    # a projection that rounds the other way is one ulp (<= 2^-7 of it) off and
+    # moves both members of its rotated pair by up to that; hi itself rounds
+    # by half an ulp: 1.5 * 2^-7 of the pair's larger member
+    scale = x.abs().amax(-1, keepdim=True).expand(-1, -1, 64).reshape(m, n)
+    got = hi.float().cpu()
+    worst = ((got - want).abs() / (2 ** -7 * scale + 1e-6)).max().item()
+    assert worst <= 1.5, worst
+    got[:, :rot] += lo.float().cpu()[:, :rot]
+    exact = ((got - want).abs() <= 2 ** -14 * scale + 1e-6).float().mean().item()
+    assert exact > 0.99, exact                # all but the projections that round the other way
+    assert (lo.cpu()[:, rot:] == 7.0).all()
+    # SiLU(gate) * up from the same weight's halves
+    wg, wu = w[:, :n // 2].contiguous(), w[:, n // 2:].contiguous()
+    got = ops.linear_silu_mul(a.cuda(), ops.pack_gate_up(wg.cuda(), wu.cuda()))
+    gate = torch.nn.functional.silu(proj[:, :n // 2]).to(BF16).float()
+    up = proj[:, n // 2:]
+    _close(got, (gate * up).to(BF16), proj[:, :n // 2] * up, up * gate)
+    assert math.isfinite(got.float().abs().max().item())

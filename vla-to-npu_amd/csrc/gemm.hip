@@ -39,90 +39,11 @@
 //    own L2): neighbouring tiles share A rows in that XCD's L2.
 #include <mutex>
 
-#include "svla_common.h"
+#include "gemm_args.h"
+
+using namespace svla_gemm;
 
 namespace {
-
-enum AMode { A_DENSE = 0, A_PSHUF = 1, A_PATCH = 2 };
-enum Epi { EPI_STORE = 0, EPI_ROPE = 1, EPI_SILU = 2, EPI_EULER = 3 };
-
-struct GemmArgs {
-  const bf16* a;
-  long lda;
-  // A_PSHUF: source [n_img, grid*grid, hidden], shuffle factor `scale`
-  int g_grid, g_hidden, g_scale;
-  // A_PATCH: images [n_img, chans, img, img], patch size
-  int p_chans, p_img, p_patch;
-  const bf16* b;
-  long ldb;
-  void* c;
-  long ldc;
-  int M, N, K;
-  float alpha;
-  const bf16* bias;
-  const float* bias_f32;
-  const bf16* res;
-  long ldr;
-  const bf16* rowadd;  // added after rounding: rowadd[(m % rowadd_period) * N + n]
-  int rowadd_period;
-  int out_f32;
-  const float* rope_cos;
-  const float* rope_sin;
-  int rope_cols;
-  int rope_period;
-  bf16* c_lo;  // ROPE (optional): o - bf16(o) of every rotated column, layout of c
-  float* x_f32;
-  long ldx;
-  bf16* x_bf16;
-  long ldxb;
-  float dt;
-  // output row remap: row m is stored at (m / c_rpg) * c_gstride + m % c_rpg
-  // (c_rpg == 0: identity).  Lets the connector write each sample's image
-  // tokens straight into its slot of the [B, prefix_len, H] prefix buffer.
-  int c_rpg;
-  long c_gstride;
-  // fused RMSNorm of the A rows: a = bf16((x * r) * w[k]), r = 1 / sqrt(mean(x^2) + eps)
-  const bf16* norm_w;
-  float norm_eps;
-  // skinny split-K (gridDim.z > 1): fp32 partial tiles [tile][split][BM * BN]
-  // and one arrival counter per output tile (zero between calls)
-  float* ws;
-  unsigned* ws_cnt;
-  // persistent wide kernel: the tile grid (its launch grid is one workgroup per
-  // CU); w_cn > 0: each XCD keeps w_cn column blocks (see xcd_tile), else the
-  // grouped order of tile_coords
-  int tiles_m, tiles_n, w_cn;
-  // slab-blocked operands / output of the wide kernel: element (row, k) of a
-  // blocked [rows, K] matrix sits at (k / 32) * rows * 32 + row * 32 + k % 32,
-  // so the 16 rows x 32 columns an LDS-DMA instruction fetches are one
-  // contiguous kilobyte (the row-major layout gives 16 separate 64-byte pieces)
-  int a_blk, b_blk, c_blk;
-};
-
-__device__ __forceinline__ long crow(const GemmArgs& p, int m) {
-  if (p.c_rpg <= 0) return m;
-  const int g = m / p.c_rpg;
-  return (long)g * p.c_gstride + (m - g * p.c_rpg);
-}
-
-template <int ACT>
-__device__ __forceinline__ float apply_act(float v) {
-  if constexpr (ACT == SVLA_ACT_GELU_TANH) return gelu_tanh_f(v);
-  else if constexpr (ACT == SVLA_ACT_GELU_ERF) return gelu_erf_f(v);
-  else if constexpr (ACT == SVLA_ACT_SILU) return silu_f(v);
-  else return v;
-}
-
-__device__ __forceinline__ void store_bf16x4(bf16* dst, const float v[4]) {
-  bf16x4 o;
-  o[0] = f2bf(v[0]); o[1] = f2bf(v[1]); o[2] = f2bf(v[2]); o[3] = f2bf(v[3]);
-  *reinterpret_cast<bf16x4*>(dst) = o;
-}
-
-__device__ __forceinline__ void load_bf16x4(const bf16* src, float v[4]) {
-  bf16x4 t = *reinterpret_cast<const bf16x4*>(src);
-  v[0] = bf2f(t[0]); v[1] = bf2f(t[1]); v[2] = bf2f(t[2]); v[3] = bf2f(t[3]);
-}
 
 // ---- epilogues: 4 consecutive (packed) columns of one row ------------------
 // Split in two so that a kernel issues the loads of a whole column tile's
@@ -300,34 +221,6 @@ __device__ __forceinline__ bf16x8 load_a(const GemmArgs& p, int m, int k) {
 
 constexpr int BK = 64;
 constexpr int LDS_STRIDE = BK + 8;  // elements; +16 bytes of padding per row
-constexpr int kNumXCD = 8;
-
-// Maps the hardware workgroup id so that consecutive logical tiles share an
-// XCD (the hardware deals workgroups round-robin over the 8 XCDs).
-__device__ __forceinline__ int xcd_remap(int bid, int total) {
-  const int per = total / kNumXCD;
-  const int full = per * kNumXCD;
-  if (bid >= full) return bid;
-  return (bid % kNumXCD) * per + bid / kNumXCD;
-}
-
-// Logical tile -> (row block, column block) in groups of kGroupRows row
-// blocks: consecutive tiles walk down a group's rows, then across its
-// columns, so the workgroups that run together on one XCD cover a compact
-// rows x columns patch and share both their A row panels and their weight
-// column panels in that XCD's L2.  (Row-major order makes a concurrent set
-// span every column block, i.e. the whole weight matrix, which does not fit.)
-constexpr int kGroupRows = 8;
-__device__ __forceinline__ void tile_coords(int t, int gm, int gn, int& tm, int& tn) {
-  const int per_group = kGroupRows * gn;
-  const int group = t / per_group;
-  const int first = group * kGroupRows;
-  const int rows = min(gm - first, kGroupRows);
-  const int r = t - group * per_group;
-  tm = first + r % rows;
-  tn = r / rows;
-}
-
 // Persistent wide kernel, column-resident order (w_cn > 0): the XCDs form
 // tiles_n / w_cn column groups, and XCD x keeps the w_cn column blocks of its
 // group (their weight panels stay in its L2 for the whole launch) and walks
@@ -2413,6 +2306,25 @@ int pick_split(int tiles, int K, int bm, int bn) {
   return max(S, 1);
 }
 
+// Problems that stay on the 32-row small tiles and the 16-column skinny tile
+// although the K-split line-DMA kernels (gemm_stream.hip) could take them:
+// their 1 to 2 us lower fixed cost wins while the grid leaves CUs idle.
+// MI355X, graph replay, these / stream: plain within two 32x32 tiles per CU --
+// O 241x960x960 5.2 / 7.1 us, down 241x960x2560 8.2 / 12.7, O 400x720x960
+// 5.9 / 7.2, down 439x960x2560 10.9 / 12.8; RoPE / SiLU within one 32x64 tile
+// per CU -- 241x1600x960 6.2 / 7.7, 400x960x720 6.1 / 7.0, but 330x1600x720
+// (275 tiles) 7.8 / 7.0 and 400x1600x720 (325) 7.9 / 7.2; up to 64 rows the
+// 16-column skinny tile -- 50x960x720 5.1 / 6.3, 50x4096x720 5.6 / 6.1, but
+// 128x1600x960 8.3 / 7.6 and 128x5120x960 9.6 / 6.9.
+bool small_range(int M, int N, int K, int epi) {
+  auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  const bool paired = epi == EPI_ROPE || epi == EPI_SILU;
+  if (M > 512 || K < LBK) return K < LBK;
+  if (!paired) return tiles(32, 32) <= 2 * kNumCU;
+  if (M <= 64) return tiles(64, 16) <= kNumCU;
+  return M > 128 && tiles(32, 64) <= kNumCU;
+}
+
 template <int AMODE, bool NORM>
 int dispatch(const GemmArgs& p, int epi, int act, TileId t, dim3 grid, hipStream_t s) {
   int rc;
@@ -2456,6 +2368,11 @@ int run_gemm(GemmArgs& p, int epi, int act, hipStream_t s, WsKind wk = WS_ALLOCA
   const bool wide_rows_ok = !p.out_f32 && p.N % 8 == 0 && p.ldc % 8 == 0 &&
                             (!p.res || (p.ldr % 8 == 0 && svla_aligned16(p.res)));
   const TileCfg t = pick_tile(p.M, p.N, p.K, epi, plain, wide_rows_ok, AMODE == A_DENSE);
+  // the K-split line-DMA kernels take the mid-size dense problems (everything
+  // but the small tiles' and the 256x256 kernel's own ranges)
+  if (AMODE == A_DENSE && g_force_tile < 0 && t.id != W256 && !small_range(p.M, p.N, p.K, epi) &&
+      stream_takes(p, epi))
+    return stream_run(p, epi, act, s);
   if (p.norm_w && p.K > 2048) return SVLA_EINVAL;  // the gain vector is staged in LDS (<= 2048)
   // a pipelined kernel needs one full K stage, the wide one whole 4-step
   // rounds of at least 8 steps (a strictly forced tile may violate either:
@@ -2535,6 +2452,15 @@ int svla_gemm_tile_choice(int m, int n, int k, int act) {
   if (m <= 0 || n <= 0 || k <= 0 || act < 0 || act > SVLA_ACT_SILU) return SVLA_EINVAL;
   (void)act;  // the choice depends on the epilogue kind, not on the activation
   return (int)pick_tile(m, n, k, EPI_STORE, true, n % 8 == 0, true).id;
+}
+
+int svla_gemm_stream_choice(int m, int n, int k, int paired) {
+  if (m <= 0 || n <= 0 || n % (paired ? 64 : 8) || k < 8 || k % 8) return SVLA_EINVAL;
+  const int epi = paired ? EPI_ROPE : EPI_STORE;
+  if (g_force_tile >= 0 || pick_tile(m, n, k, epi, !paired, true, true).id == W256 ||
+      small_range(m, n, k, epi))
+    return 0;
+  return stream_tile(m, n, k, epi);
 }
 
 int svla_gemm_set_split(int splits) {
