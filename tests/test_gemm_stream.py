@@ -137,3 +137,48 @@ def test_paired_epilogues(m, n, k):
     up = proj[:, n // 2:]
     _close(got, (gate * up).to(BF16), proj[:, :n // 2] * up, up * gate)
     assert math.isfinite(got.float().abs().max().item())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,grid,hidden,scale,n_out", [
+    (1, 32, 768, 4, 960), (3, 32, 768, 4, 960), (5, 32, 768, 4, 960), (9, 32, 768, 4, 960),
+    (17, 32, 768, 4, 960), (33, 32, 768, 4, 960), (2, 24, 200, 3, 72), (5, 8, 104, 2, 968)])
+def test_connector(n, grid, hidden, scale, n_out):
+    """Pixel-shuffle gather, unsplit and with K split over workgroups, into
+    plain rows and into each sample's slot of a larger buffer (whose other
+    rows stay as they were)."""
+    from smolvla import ops
+    g = torch.Generator().manual_seed(n * grid + hidden)
+    x = torch.randn(n, grid * grid, hidden, generator=g).to(BF16)
+    K, per = hidden * scale * scale, (grid // scale) ** 2
+    w = (torch.randn(K, n_out, generator=g) * 0.05).to(BF16)
+    t = x.view(n, grid // scale, scale, grid // scale, scale, hidden).permute(0, 1, 3, 2, 4, 5)
+    want = (t.reshape(n * per, K).float() @ w.float()).to(BF16)
+    wp = ops.pack_weight(w.cuda())
+    _close(ops.connector(x.cuda(), wp, scale), want)
+    buf = torch.full((n * (per + 9), n_out), 3.0, dtype=BF16, device="cuda")
+    ops.connector(x.cuda(), wp, scale, out=buf, rows_per_sample=per, sample_stride=per + 9)
+    got = buf.cpu().view(n, per + 9, n_out)
+    _close(got[:, :per].reshape(n * per, n_out), want)
+    assert (got[:, per:] == 3.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,chans,image,patch,embed", [
+    (1, 3, 512, 16, 768), (2, 3, 512, 16, 768), (7, 3, 512, 16, 768), (3, 1, 72, 8, 72),
+    (2, 3, 120, 24, 200)])
+@pytest.mark.parametrize("pos", [True, False])
+def test_patch_embed(n, chans, image, patch, embed, pos):
+    from smolvla import ops
+    g = torch.Generator().manual_seed(n * image + embed)
+    x = (torch.rand(n, chans, image, image, generator=g) * 2 - 1).to(BF16)
+    w = (torch.randn(embed, chans, patch, patch, generator=g) * 0.05).to(BF16)
+    b = torch.randn(embed, generator=g).to(BF16)
+    G = image // patch
+    table = torch.randn(G * G, embed, generator=g).to(BF16) if pos else None
+    y = torch.nn.functional.conv2d(x.float(), w.float(), b.float(), stride=patch)
+    y = y.flatten(2).transpose(1, 2).to(BF16).float()
+    want = (y + table.float()).to(BF16) if pos else y.to(BF16)
+    got = ops.patch_embed(x.cuda(), w.reshape(embed, -1).cuda(), b.cuda(),
+                          table.cuda() if pos else None, patch)
+    _close(got.view(n, G * G, embed), want, y)

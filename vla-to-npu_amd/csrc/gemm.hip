@@ -2136,11 +2136,8 @@ TileCfg pick_tile(int M, int N, int K, int epi, bool plain, bool wide_rows_ok, b
   // + SiLU 7712x5120x960 93.4 (116.4 register-staged); a grid under one
   // 128x128 tile per CU takes the 64x64 line tile (the cross K/V projection
   // 7712x320x320: 9.4 -> 7.6 us).
-  // The gathers from M = 4096 (the batch-32 patch embedding 98304x768x768
-  // and pixel-shuffle connector 6144x960x12288), measured on MI355X with
-  // graph replay: the register-staged 128x128 kernel -- patch 311 -> 219 us,
-  // connector 310 -> 211 us against the 64x64 line tile the M >= 3072 rule
-  // below would take (the 128x128 LDS-DMA pipeline: 235 / 210 us)
+  // (gathers reach this choice only with outputs that the gather kernels of
+  // gemm_stream.hip do not take)
   if (!dense && M >= 4096) return tile_dims(T128);
   if (dense && M >= 4096) {
     if (!line_ok) return tile_dims(T128);
@@ -2373,6 +2370,12 @@ int run_gemm(GemmArgs& p, int epi, int act, hipStream_t s, WsKind wk = WS_ALLOCA
   if (AMODE == A_DENSE && g_force_tile < 0 && t.id != W256 && !small_range(p.M, p.N, p.K, epi) &&
       stream_takes(p, epi))
     return stream_run(p, epi, act, s);
+  if (AMODE != A_DENSE && g_force_tile < 0 && epi == EPI_STORE && gather_takes(p)) {
+    // (a capture that comes before the workspace exists runs unsplit)
+    const SplitWs* w = (long)p.M * p.N * 2 <= (long)kWsFloats && g_force_split != 1 ? split_ws(s) : nullptr;
+    p.ws = w ? w->part : nullptr;
+    return gather_run(p, AMODE, s, (long)kWsFloats);
+  }
   if (p.norm_w && p.K > 2048) return SVLA_EINVAL;  // the gain vector is staged in LDS (<= 2048)
   // a pipelined kernel needs one full K stage, the wide one whole 4-step
   // rounds of at least 8 steps (a strictly forced tile may violate either:

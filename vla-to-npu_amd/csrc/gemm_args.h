@@ -7,7 +7,8 @@
 namespace svla_gemm {
 
 enum AMode { A_DENSE = 0, A_PSHUF = 1, A_PATCH = 2 };
-enum Epi { EPI_STORE = 0, EPI_ROPE = 1, EPI_SILU = 2, EPI_EULER = 3 };
+// EPI_PART: fp32 partial tiles of a K split (gemm_stream.hip)
+enum Epi { EPI_STORE = 0, EPI_ROPE = 1, EPI_SILU = 2, EPI_EULER = 3, EPI_PART = 4 };
 
 struct GemmArgs {
   const bf16* a;
@@ -123,5 +124,11 @@ __attribute__((visibility("hidden"))) bool stream_takes(const GemmArgs& p, int e
 __attribute__((visibility("hidden"))) int stream_tile(int M, int N, int K, int epi);
 __attribute__((visibility("hidden"))) int stream_run(const GemmArgs& p, int epi, int act,
                                                      hipStream_t s);
+
+// The gathers (pixel shuffle, patches) on the same kernels; p.ws: room for
+// ws_floats floats of split-K partial tiles, or null.
+__attribute__((visibility("hidden"))) bool gather_takes(const GemmArgs& p);
+__attribute__((visibility("hidden"))) int gather_run(const GemmArgs& p, int amode, hipStream_t s,
+                                                     long ws_floats);
 
 }  // namespace svla_gemm

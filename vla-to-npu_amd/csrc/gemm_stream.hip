@@ -63,9 +63,43 @@ __device__ __forceinline__ int pair_col(int j) {
   return 64 * (u >> 1) + 16 * (u & 1) + (q & 15) + 32 * (q >> 4);
 }
 
-template <int BM, int BN, int WMW, int KG, int ST, int MINB, int EPI, int ACT>
+// Element offset of A[m][k] = a_row(m) + a_col(k): both gathers separate (k in
+// chunks of 8, which neither map splits; the maps are those of a_ptr in
+// gemm.hip).  Pixel shuffle: the s tokens of one patch row are adjacent, so
+// k runs through s * E contiguous elements, then jumps a token row.  Patches:
+// 8 adjacent patches give the 8-row DMA block 4 runs of 256 bytes per stage.
+template <int AMODE>
+__device__ __forceinline__ long a_row(const GemmArgs& p, int m) {
+  if constexpr (AMODE == A_DENSE) {
+    return (long)m * p.lda;
+  } else if constexpr (AMODE == A_PSHUF) {
+    const int gs = p.g_grid / p.g_scale, per = gs * gs;
+    const int img = m / per, i = m - img * per, hp = i / gs, wp = i - hp * gs;
+    return ((long)img * p.g_grid * p.g_grid + (long)p.g_scale * hp * p.g_grid + p.g_scale * wp) *
+           p.g_hidden;
+  } else {
+    const int P = p.p_patch, H = p.p_img, G = H / P, per = G * G;
+    const int img = m / per, t = m - img * per, pr = t / G, pc = t - pr * G;
+    return ((long)img * p.p_chans * H + pr * P) * H + pc * P;
+  }
+}
+template <int AMODE>
+__device__ __forceinline__ long a_col(const GemmArgs& p, int k) {
+  if constexpr (AMODE == A_DENSE) {
+    return k;
+  } else if constexpr (AMODE == A_PSHUF) {
+    const int sE = p.g_scale * p.g_hidden, t = k / sE;
+    return (long)t * p.g_grid * p.g_hidden + (k - t * sE);
+  } else {
+    const int P = p.p_patch, P2 = P * P, ch = k / P2, r = k - ch * P2, ky = r / P;
+    return ((long)ch * p.p_img + ky) * p.p_img + (r - ky * P);
+  }
+}
+
+template <int BM, int BN, int WMW, int KG, int ST, int MINB, int AMODE, int EPI, int ACT>
 __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs p) {
   constexpr bool PAIRED = EPI == EPI_ROPE || EPI == EPI_SILU;
+  static_assert(AMODE == A_DENSE || (BM % 64 == 0 && (EPI == EPI_STORE || EPI == EPI_PART)), "gathers");
   constexpr int WNW = GW / WMW / KG;                 // waves along the columns
   constexpr int WM = BM / WMW, WN = BN / WNW;        // wave tile
   constexpr int TM = WM / 16, TN = WN / 16, NF = TM + TN, NM = TM * TN;
@@ -96,7 +130,10 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
   int tm_idx, tn_idx;
   tile_coords(tile, p.tiles_m, p.tiles_n, tm_idx, tn_idx);
   const int m0 = tm_idx * BM, n0 = tn_idx * BN;
-  const int nk = (p.K + GK - 1) / GK;
+  // this workgroup's K stages: all, or split blockIdx.z of gridDim.z (EPI_PART)
+  const int nk_all = (p.K + GK - 1) / GK;
+  const int kt0 = EPI == EPI_PART ? (int)((long)nk_all * blockIdx.z / gridDim.z) : 0;
+  const int nk = EPI == EPI_PART ? (int)((long)nk_all * (blockIdx.z + 1) / gridDim.z) - kt0 : nk_all;
 
   // residual pieces of this thread's stores: requested before the K loop at one
   // workgroup per CU, after it at two (registers; the other workgroup covers)
@@ -105,10 +142,14 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       const int q = tid + i * GW * 64, r = q / PPR, c = q - r * PPR;
-      rsd[i] = ld8(p.res + (long)min(m0 + r, p.M - 1) * p.ldr + min(n0 + c * 8, p.N - 8));
+      const int m = min(m0 + r, p.M - 1), n = min(n0 + c * 8, p.N - 8);
+      rsd[i] = ld8(AMODE == A_PATCH ? p.rowadd + (long)(m % p.rowadd_period) * p.N + n
+                                    : p.res + (long)m * p.ldr + n);
     }
   };
-  if (EPI == EPI_STORE && MINB == 1 && p.res) load_res();
+  // (the patch embedding's addend is its position table)
+  const bool addend = EPI == EPI_STORE && (AMODE == A_PATCH ? p.rowadd : p.res) != nullptr;
+  if (MINB == 1 && addend) load_res();
 
   // DMA block j * 8 + wave of a stage: rows 8 blk .. + 7 of [A | W], 8 lanes
   // per 128-byte row piece, chunk c of row r in slot gswz(r, c)
@@ -119,7 +160,7 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
   for (int j = 0; j < ND; ++j) {
     const int r = min(j * GW + wave, TD - 1) * 8 + (lane >> 3);
     if (r < BM) {
-      src[j] = p.a + (long)min(m0 + r, p.M - 1) * p.lda;
+      src[j] = p.a + a_row<AMODE>(p, min(m0 + r, p.M - 1));
     } else {
       const int c = n0 + r - BM;
       src[j] = p.b + (long)min(PAIRED ? pair_col(c) : c, p.N - 1) * p.ldb;
@@ -128,7 +169,9 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
   auto dma = [&](int slot, int kt, int j) __attribute__((always_inline)) {
     if (TD % GW != 0 && j == ND - 1 && !all) return;  // wave-uniform
     // chunks past K reload the row's last one (masked before the MFMAs)
-    __builtin_amdgcn_global_load_lds((void*)(src[j] + min(kt * GK + chunk, p.K - 8)),
+    const int k = min((kt0 + kt) * GK + chunk, p.K - 8);
+    const long off = AMODE != A_DENSE && j < BM / 64 ? a_col<AMODE>(p, k) : k;  // (blocks < BM / 8: A)
+    __builtin_amdgcn_global_load_lds((void*)(src[j] + off),
                                      (lds_ptr_t)(sh + slot * STAGE + (j * GW + wave) * 512), 16, 0,
                                      0);
   };
@@ -191,7 +234,7 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
   // the last stage: fragments past K are zero in both operands
   auto mask = [&](auto RC, int h) __attribute__((always_inline)) {
     constexpr int R = decltype(RC)::value;
-    if ((nk - 1) * GK + (4 * h + g) * 8 >= p.K) {
+    if ((kt0 + nk - 1) * GK + (4 * h + g) * 8 >= p.K) {
 #pragma unroll
       for (int f = 0; f < NF; ++f) fr_[R][f] = bf16x8{};
     }
@@ -297,6 +340,17 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
         acc[i] += *reinterpret_cast<const f32x4*>(ex + i * 256 + lane * 4);
     __syncthreads();  // exchange read: the space takes the output
   }
+  if constexpr (EPI == EPI_PART) {
+    // fp32 partial tile of this split, [split][M][N]
+    float* part = p.ws + (long)blockIdx.z * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+      const int t = i % TN, m = m0 + wm * WM + i / TN * 16 + fr, n = ccol(t);
+      if ((KG == 2 && (t < H0) != (kg == 0)) || m >= p.M || n >= p.N) continue;
+      *reinterpret_cast<f32x4*>(part + (long)m * p.N + n) = acc[i];
+    }
+    return;
+  }
   auto stage = [&](int row, int col, const float (&v)[4], int half) __attribute__((always_inline)) {
     bf16x4 o;
 #pragma unroll
@@ -358,7 +412,7 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
   };
   if (KG == 1 || kg == 0) finish(I0{});
   else finish(I1{});
-  if (EPI == EPI_STORE && MINB > 1 && p.res) load_res();
+  if (MINB > 1 && addend) load_res();
   __syncthreads();
   // whole 16-byte pieces of consecutive columns, row by row
 #pragma unroll
@@ -368,15 +422,41 @@ __global__ __launch_bounds__(GW * 64, 2 * MINB) void gemm_stream_kernel(GemmArgs
     const int n = EPI == EPI_SILU ? n0 / 2 + c * 8 : EPI == EPI_ROPE ? pair_col(n0 + c * 8) : n0 + c * 8;
     if (q >= BM * PPR || m >= p.M || n0 * BNO / BN + c * 8 >= p.N * BNO / BN) continue;
     bf16x8 o = *reinterpret_cast<const bf16x8*>(sh + r * LDO + c * 8);
-    if (EPI == EPI_STORE && p.res) {
+    if (addend) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = f2bf(bf2f(o[e]) + bf2f(rsd[i][e]));
     }
-    st8(reinterpret_cast<bf16*>(p.c) + (long)m * p.ldc + n, o);
+    st8(reinterpret_cast<bf16*>(p.c) + (AMODE == A_PSHUF ? crow(p, m) : (long)m) * p.ldc + n, o);
     if (EPI == EPI_ROPE && p.c_lo && n < p.rope_cols)
       st8(p.c_lo + (long)m * p.ldc + n,
           *reinterpret_cast<const bf16x8*>(sh + BM * LDO + r * LDO + c * 8));
   }
+}
+
+// Sums the K splits' partial tiles in split order and finishes the rows: bias,
+// one rounding, the position table, the row remap.  One thread per 8 columns.
+__global__ __launch_bounds__(256) void stream_reduce_kernel(GemmArgs p, int splits) {
+  const int per = p.N / 8;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.M * per) return;
+  const int m = i / per, n = (i - m * per) * 8;
+  const float* src = p.ws + (long)m * p.N + n;
+  const long step = (long)p.M * p.N;
+  f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+#pragma unroll 4
+  for (int z = 0; z < splits; ++z) {
+    a += *reinterpret_cast<const f32x4*>(src + z * step);
+    b += *reinterpret_cast<const f32x4*>(src + z * step + 4);
+  }
+  bf16x8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float v = (e < 4 ? a[e & 3] : b[e & 3]) * p.alpha;
+    if (p.bias) v += bf2f(p.bias[n + e]);
+    if (p.rowadd) v = rbf(v) + bf2f(p.rowadd[(long)(m % p.rowadd_period) * p.N + n + e]);
+    o[e] = f2bf(v);
+  }
+  st8(reinterpret_cast<bf16*>(p.c) + crow(p, m) * p.ldc + n, o);
 }
 
 template <int BM, int BN, int WMW, int KG, int ST, int MINB>
@@ -385,7 +465,7 @@ int launch_stream(GemmArgs p, int epi, int act, hipStream_t s) {
   p.tiles_n = (p.N + BN - 1) / BN;
   const dim3 grid(p.tiles_m * p.tiles_n), block(GW * 64);
 #define SVLA_STREAM(E, A) \
-  hipLaunchKernelGGL((gemm_stream_kernel<BM, BN, WMW, KG, ST, MINB, E, A>), grid, block, 0, s, p)
+  hipLaunchKernelGGL((gemm_stream_kernel<BM, BN, WMW, KG, ST, MINB, A_DENSE, E, A>), grid, block, 0, s, p)
   if (epi == EPI_STORE) {
     if (act == SVLA_ACT_GELU_TANH) SVLA_STREAM(EPI_STORE, SVLA_ACT_GELU_TANH);
     else if (act == SVLA_ACT_GELU_ERF) SVLA_STREAM(EPI_STORE, SVLA_ACT_GELU_ERF);
@@ -402,6 +482,30 @@ int launch_stream(GemmArgs p, int epi, int act, hipStream_t s) {
   return 0;
 }
 
+// The gathers, K split over `splits` workgroups per tile (1: none).
+template <int BM, int BN, int WMW, int KG, int ST, int MINB>
+int launch_gather(GemmArgs p, int amode, int splits, hipStream_t s) {
+  p.tiles_m = (p.M + BM - 1) / BM;
+  p.tiles_n = (p.N + BN - 1) / BN;
+  const dim3 grid(p.tiles_m * p.tiles_n, 1, splits), block(GW * 64);
+#define SVLA_GATHER(A, E) \
+  hipLaunchKernelGGL((gemm_stream_kernel<BM, BN, WMW, KG, ST, MINB, A, E, 0>), grid, block, 0, s, p)
+  if (amode == A_PSHUF) {
+    if (splits > 1) SVLA_GATHER(A_PSHUF, EPI_PART);
+    else SVLA_GATHER(A_PSHUF, EPI_STORE);
+  } else {
+    if (splits > 1) SVLA_GATHER(A_PATCH, EPI_PART);
+    else SVLA_GATHER(A_PATCH, EPI_STORE);
+  }
+#undef SVLA_GATHER
+  SVLA_CHECK_LAUNCH();
+  if (splits > 1) {
+    hipLaunchKernelGGL(stream_reduce_kernel, dim3((p.M * (p.N / 8) + 255) / 256), dim3(256), 0, s, p,
+                       splits);
+    SVLA_CHECK_LAUNCH();
+  }
+  return 0;
+}
 
 // The configurations and what they cost (microseconds): a launch, one round of
 // workgroups over the chip's slots (256 CUs x MINB), and each 64-deep stage of
@@ -430,25 +534,53 @@ const StreamCfg kStream[] = {
     {256, 128, 1, true, 0.42f, 7.68f, 0.635f, 0.f, launch_stream<256, 128, 4, 1, 3, 1>},
 };
 
+// microseconds of a problem on configuration c, K split over `splits`
+template <class C>
+double stream_cost(const C& c, int M, int N, int K, int splits) {
+  const long nk = ((K + GK - 1) / GK + splits - 1) / splits;
+  const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * splits;
+  const long full = tiles / (256L * c.wg), rest = tiles % (256L * c.wg);
+  const bool single = c.wg == 2 && rest > 0 && rest <= 256;
+  return c.launch + c.round * (full + (rest > 0)) +
+         nk * ((double)c.stage * (full + (rest > 0 && !single)) + (single ? c.stage1 : 0.f));
+}
+
 const StreamCfg& pick_stream(int M, int N, int K, int epi) {
   const bool paired = epi == EPI_ROPE || epi == EPI_SILU;
-  const long nk = (K + GK - 1) / GK;
   const StreamCfg* best = nullptr;
   double best_us = 0;
   for (const StreamCfg& c : kStream) {
     if (paired && !c.paired) continue;
-    const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-    const long full = tiles / (256L * c.wg), rest = tiles % (256L * c.wg);
-    const bool single = c.wg == 2 && rest > 0 && rest <= 256;
-    const double us = c.launch + c.round * (full + (rest > 0)) +
-                      nk * ((double)c.stage * (full + (rest > 0 && !single)) +
-                            (single ? c.stage1 : 0.f));
+    const double us = stream_cost(c, M, N, K, 1);
     if (!best || us < best_us) {
       best = &c;
       best_us = us;
     }
   }
   return *best;
+}
+
+// The gathers' configurations (costs as kStream's).
+struct GatherCfg {
+  int bm, bn, wg;
+  float launch, round, stage, stage1;
+  int (*run)(GemmArgs, int, int, hipStream_t);
+};
+const GatherCfg kGather[] = {
+    {64, 64, 1, 3.46f, 0.87f, 0.193f, 0.f, launch_gather<64, 64, 4, 2, 4, 1>},
+    {64, 96, 2, 2.67f, 2.26f, 0.507f, 0.270f, launch_gather<64, 96, 4, 2, 3, 2>},
+    {64, 160, 1, 1.90f, 3.79f, 0.375f, 0.f, launch_gather<64, 160, 4, 2, 4, 1>},
+    {128, 128, 1, 0.95f, 5.89f, 0.388f, 0.f, launch_gather<128, 128, 4, 2, 4, 1>},
+    {128, 192, 1, 0.00f, 5.94f, 0.520f, 0.f, launch_gather<128, 192, 2, 1, 3, 1>},
+    {192, 128, 1, 0.60f, 6.27f, 0.531f, 0.f, launch_gather<192, 128, 4, 1, 3, 1>},
+    {256, 128, 1, 0.42f, 7.68f, 0.635f, 0.f, launch_gather<256, 128, 4, 1, 3, 1>},
+};
+constexpr int kMaxSplits = 12;
+// A split's partial tiles: the reduction launch, and their fp32 write and read
+// (connector at 1 to 32 images, measured beyond the tiles' own cost: 6.4 us for
+// 6 MB, 8.3 for 12, 16-20 for 32).
+double split_cost(int M, int N, int splits) {
+  return splits == 1 ? 0.0 : 4.0 + 8e-6 * M * N * splits / 2.3;
 }
 
 }  // namespace
@@ -468,6 +600,37 @@ bool stream_takes(const GemmArgs& p, int epi) {
 int stream_tile(int M, int N, int K, int epi) {
   const StreamCfg& c = pick_stream(M, N, K, epi);
   return c.bm * 1000 + c.bn;
+}
+
+bool gather_takes(const GemmArgs& p) {
+  return p.M >= 64 && p.K >= GK && p.N % 8 == 0 && p.ldc % 8 == 0 && !p.out_f32 && !p.bias_f32 &&
+         !p.res && !p.norm_w;
+}
+
+// Batched gathers take large tiles, unsplit; a few images' connector has tens
+// of tiles and K = 12288, so its K is split over workgroups as far as the
+// workspace of `ws_floats` floats holds the partial tiles.  MI355X, graph
+// replay, before (64x64 line tile, register-staged 128x128 or split skinny
+// tiles) / now: connector of 1 image 21.6 / 13.8 us, 3 images 40.3 / 19.5, 9
+// images 102 / 32, 32 images 133 / 64, 96 images 250 / 158; patch embedding of
+// 1 image 12.3 / 8.7, 7 images 26.7 / 16.6, 96 images 245 / 174.
+int gather_run(const GemmArgs& p, int amode, hipStream_t s, long ws_floats) {
+  const GatherCfg* best = nullptr;
+  int splits = 1;
+  double best_us = 0;
+  const int nk = (p.K + GK - 1) / GK;
+  for (const GatherCfg& c : kGather)
+    for (int z = 1; z <= kMaxSplits && z * 4 <= nk; ++z) {
+      if (z > 1 && (!p.ws || (long)z * p.M * p.N > ws_floats)) break;
+      const double us = stream_cost(c, p.M, p.N, p.K, z) + split_cost(p.M, p.N, z);
+      if (!best || us < best_us) {
+        best = &c;
+        best_us = us;
+        splits = z;
+      }
+    }
+  if (!best) return kGather[0].run(p, amode, 1, s);
+  return best->run(p, amode, splits, s);
 }
 
 int stream_run(const GemmArgs& p, int epi, int act, hipStream_t s) {
