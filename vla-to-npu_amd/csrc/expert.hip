@@ -96,7 +96,8 @@ enum XStat { XS_OK = 0, XS_TIMEOUT = 1, XS_TEAM = 2 };
 struct XPhase {
   int kind, epi, act, a_f32;
   int M, N, K, units, col_tiles;
-  int row_groups, group_tiles;  // GEMM unit = (column tile, group of row tiles)
+  int row_groups, group_tiles;  // GEMM unit = (column group, group of row tiles)
+  int cts;                      // 16-column tiles per column group (1 or 2)
   // GEMM: C[M, N] = epilogue(norm(A)[M, K] . W[N, K]^T)
   const void* a;
   int lda;
@@ -240,9 +241,15 @@ __device__ bool wait_phase(const XArgs& g, int row, unsigned target) {
 }
 
 // ---- GEMM units ---------------------------------------------------------------
+// NT: row tiles of a unit (P.group_tiles: 1, 2 or 4), counted from its first;
+// compile-time, like the column tiles CT, so that loads, normalisation and
+// MFMAs are straight runs (with run-time bounds every tile was a branch whose
+// region ended in a wait: the MFMA step of norm + gate|up took 1.15 us, 0.6 as
+// a straight run).
+template <int NT>
 struct GemmRegs {
-  bf16x8 fx[XKS][4];  // activations: this wave's k-steps x 4 row tiles
-  float ss[4];        // norm: this lane's row sums of squares (rows tm*16 + fr)
+  bf16x8 fx[XKS][NT];  // activations: this wave's k-steps x row tiles
+  float ss[NT];        // norm: this lane's row sums of squares
 };
 
 // LDS image of one wave's weight fragments: k-step j of the unit's 16 rows,
@@ -288,29 +295,31 @@ __device__ __forceinline__ void wave_krange(int K, int wave, int& ks0, int& kcnt
   kcnt = max(0, min(per, nks - ks0));
 }
 
-// Weight fragments of column tile ct for this wave's k-steps, streamed into
+// Weight fragments of column group cg for this wave's k-steps, streamed into
 // the wave's own LDS region by LDS-DMA (no registers held while they fly;
 // only this wave reads them, after its own vmcnt wait).  Lane l fetches row
 // l / 4 (through the paired-tile row map), chunk wswz(row, l % 4).  Only the
 // wave's own k-steps are requested: a CU holds a bounded number of misses in
 // flight, and repeated requests of one line use them up.  Chunks past K hold
 // other weights: the activations there are zero.
-__device__ __forceinline__ void dma_w(int epi, const bf16* W, int N, int K, int ldw, int ct,
+__device__ __forceinline__ void dma_w(int epi, const bf16* W, int N, int K, int ldw, int cts, int cg,
                                       bf16* sw) {
   const int lane = tidx() & 63;
   const int wave = wave_id();
   int ks0, kcnt;
   wave_krange(K, wave, ks0, kcnt);
-  const int base = tile_base(epi, ct);
   const int r = lane >> 2;
-  const int row = paired(epi) ? base + (r & 7) + (r >> 3) * 32 : min(base + r, N - 1);
   const int c8 = wswz(r, lane & 3) * 8;
-  const bf16* src = W + (long)row * ldw;
+  for (int c = 0; c < cts; ++c) {  // uniform; cts * kcnt <= XKS
+    const int base = tile_base(epi, cg * cts + c);
+    const int row = paired(epi) ? base + (r & 7) + (r >> 3) * 32 : min(base + r, N - 1);
+    const bf16* src = W + (long)row * ldw;
 #pragma unroll
-  for (int j = 0; j < XKS; ++j) {
-    if (j >= kcnt) break;  // wave-uniform
-    __builtin_amdgcn_global_load_lds((void*)(src + min((ks0 + j) * 32 + c8, K - 8)),
-                                     (lds_ptr_t)(sw + j * XWSTEP), 16, 0, 0);
+    for (int j = 0; j < XKS; ++j) {
+      if (j >= kcnt) break;  // wave-uniform
+      __builtin_amdgcn_global_load_lds((void*)(src + min((ks0 + j) * 32 + c8, K - 8)),
+                                       (lds_ptr_t)(sw + (c * kcnt + j) * XWSTEP), 16, 0, 0);
+    }
   }
 }
 
@@ -328,33 +337,34 @@ __device__ __forceinline__ void dma_gain(const bf16* norm_w, int K, bf16* gain) 
 // Activation fragments (rows 0..63, clamped to M - 1) of this wave's k-steps
 // (only those: steps past the range are never requested); k past K reads as
 // zero.
-__device__ __forceinline__ void load_x(CPhase& P, GemmRegs& r, int t0, int t1) {
+template <int NT>
+__device__ __forceinline__ void load_x(CPhase& P, GemmRegs<NT>& r, int t0) {
   const int lane = tidx() & 63;
   const int wave = wave_id();
   const int fr = lane & 15, fk = (lane >> 4) * 8;
   int ks0, kcnt;
   wave_krange(P.K, wave, ks0, kcnt);
-  unsigned rows[4];
+  unsigned rows[NT];
 #pragma unroll
-  for (int tm = 0; tm < 4; ++tm) rows[tm] = (unsigned)min(tm * 16 + fr, P.M - 1);
+  for (int tm = 0; tm < NT; ++tm) rows[tm] = (unsigned)min((t0 + tm) * 16 + fr, P.M - 1);
   if (P.a_f32) {
     // fp32 A (the Euler state into action_in, K <= 32: one k-step, wave 0),
     // rounded to bf16 on the way in (only k-step 0 exists)
 #pragma unroll
-    for (int tm = 0; tm < 4; ++tm) r.fx[0][tm] = bf16x8{};
+    for (int tm = 0; tm < NT; ++tm) r.fx[0][tm] = bf16x8{};
     if (kcnt > 0) {
       const int k = ks0 * 32 + fk;
       // every load issued before any use (a use right after its load would
       // make each load a round trip of its own)
-      f32x4 lo[4], hi[4];
+      f32x4 lo[NT], hi[NT];
 #pragma unroll
-      for (int tm = 0; tm < 4; ++tm) {
+      for (int tm = 0; tm < NT; ++tm) {
         const float* src = static_cast<const float*>(P.a) + (rows[tm] * (unsigned)P.lda + (unsigned)min(k, P.K - 8));
         lo[tm] = ldgf4(src);
         hi[tm] = ldgf4(src + 4);
       }
 #pragma unroll
-      for (int tm = 0; tm < 4; ++tm) {
+      for (int tm = 0; tm < NT; ++tm) {
         bf16x8 t;
 #pragma unroll
         for (int i = 0; i < 4; ++i) { t[i] = f2bf(lo[tm][i]); t[4 + i] = f2bf(hi[tm][i]); }
@@ -370,14 +380,13 @@ __device__ __forceinline__ void load_x(CPhase& P, GemmRegs& r, int t0, int t1) {
     for (int j = 0; j < XKS; ++j) {
       if (j >= kcnt) break;  // wave-uniform: no request past the wave's range
 #pragma unroll
-      for (int tm = 0; tm < 4; ++tm) {
-        if (tm < t0 || tm >= t1) continue;  // wave-uniform: another unit's rows
-        r.fx[j][tm] = ldg8(static_cast<const bf16*>(P.a) + (((unsigned)(ks0 + j) * 4u + tm) * 64u + lane) * 8u);
+      for (int tm = 0; tm < NT; ++tm) {
+        r.fx[j][tm] = ldg8(static_cast<const bf16*>(P.a) + (((unsigned)(ks0 + j) * 4u + t0 + tm) * 64u + lane) * 8u);
       }
     }
   }
 #pragma unroll
-  for (int tm = 0; tm < 4; ++tm) r.ss[tm] = 0.f;
+  for (int tm = 0; tm < NT; ++tm) r.ss[tm] = 0.f;
   if (P.norm_w) {
     // per-row sums of squares of the raw activations (norm_x applies
     // 1 / rms and the gains once the waves' sums have met); the activations
@@ -389,8 +398,7 @@ __device__ __forceinline__ void load_x(CPhase& P, GemmRegs& r, int t0, int t1) {
     for (int j = 0; j < XKS; ++j) {
       if (j >= kcnt) continue;  // wave-uniform
 #pragma unroll
-      for (int tm = 0; tm < 4; ++tm) {
-        if (tm < t0 || tm >= t1) continue;  // wave-uniform
+      for (int tm = 0; tm < NT; ++tm) {
         const bf16x8 x = r.fx[j][tm];
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
@@ -404,29 +412,29 @@ __device__ __forceinline__ void load_x(CPhase& P, GemmRegs& r, int t0, int t1) {
 
 // Epilogue work item of thread tid in a unit: tile row ml, 4-column group
 // gi, first packed column n; `on` false if the thread has none.
+// `pr` is its row of the LDS partial tiles: the row inside the unit, plus 32
+// in the second column tile (a unit of two has at most 32 rows).
 struct EpiItem {
-  int ml, n, gi;
+  int ml, n, gi, pr;
   bool on;
 };
 
-__device__ __forceinline__ bool vt_unit(CPhase& P, int ct) {
-  return P.vt && tile_base(P.epi, ct) >= P.rope_cols;
+__device__ __forceinline__ bool vt_unit(CPhase& P, int cg) {
+  return P.vt && tile_base(P.epi, cg * P.cts) >= P.rope_cols;
 }
 
-__device__ __forceinline__ EpiItem epi_item(CPhase& P, int ct, int t0, int t1) {
+__device__ __forceinline__ int part_row(int c, int m, int t0) { return c * 32 + m - t0 * 16; }
+
+__device__ __forceinline__ EpiItem epi_item(CPhase& P, int cg, int t0, int t1) {
   const int tid = tidx();
   EpiItem it{};
-  const int base = tile_base(P.epi, ct);
-  if (paired(P.epi)) {
-    it.ml = tid >> 1;
-    it.gi = tid & 1;
-    it.on = tid < XBM * 2 && it.ml < P.M;
-  } else {
-    it.ml = tid >> 2;
-    it.gi = tid & 3;
-    it.on = tid < XBM * 4 && it.ml < P.M;
-  }
-  it.n = base + it.gi * 4;
+  const int sh = paired(P.epi) ? 1 : 2;  // log2 of the 4-column groups per row
+  it.pr = tid >> sh;
+  it.gi = tid & ((1 << sh) - 1);
+  const int c = P.cts == 2 ? (it.pr >> 5) & 1 : 0;
+  it.ml = t0 * 16 + (P.cts == 2 ? it.pr & 31 : it.pr);
+  it.on = it.pr < XBM && it.ml < P.M;
+  it.n = tile_base(P.epi, cg * P.cts + c) + it.gi * 4;
   if (!paired(P.epi) && it.n >= P.N) it.on = false;
   if ((it.ml >> 4) < t0 || (it.ml >> 4) >= t1) it.on = false;  // another unit's rows
   return it;
@@ -473,28 +481,29 @@ union XShared {
 // order.  The gains of the wave's k range were staged in LDS by dma_gain
 // (landed: load_x waited for every load of the wave).  Rows past M are zero
 // and stay zero.
-__device__ __forceinline__ void norm_x(CPhase& P, GemmRegs& r, const XShared& sh, int t0,
-                                       int t1) {
+template <int NT>
+__device__ __forceinline__ void norm_x(CPhase& P, GemmRegs<NT>& r, const XShared& sh, int t0) {
   const int lane = tidx() & 63, wave = wave_id();
   const int fr = lane & 15, G = lane >> 4;
   int ks0, kcnt;
   wave_krange(P.K, wave, ks0, kcnt);
-  float rs[4];
+  // lane l forms row l's scale once and the fragments' rows are shuffled out
+  // of it (a square root and two divisions per row tile and lane were most of
+  // this step: norm + Q 1.6 us of 5.1)
+  float t = 0.f;
 #pragma unroll
-  for (int tm = 0; tm < 4; ++tm) {
-    float t = 0.f;
+  for (int w = 0; w < XW; ++w) t += sh.g.ss[w][lane];
+  const float rl = 1.0f / sqrtf(t / (float)P.K + P.norm_eps);
+  float rs[NT];
 #pragma unroll
-    for (int w = 0; w < XW; ++w) t += sh.g.ss[w][tm * 16 + fr];
-    rs[tm] = 1.0f / sqrtf(t / (float)P.K + P.norm_eps);
-  }
+  for (int tm = 0; tm < NT; ++tm) rs[tm] = __shfl(rl, (t0 + tm) * 16 + fr, 64);
   const bf16* gain = sh.g.gain[wave];
 #pragma unroll
   for (int j = 0; j < XKS; ++j) {
     if (j >= kcnt) break;  // wave-uniform
     const bf16x8 gv = *reinterpret_cast<const bf16x8*>(gain + j * 32 + G * 8);
 #pragma unroll
-    for (int tm = 0; tm < 4; ++tm) {
-      if (tm < t0 || tm >= t1) continue;  // wave-uniform
+    for (int tm = 0; tm < NT; ++tm) {
       bf16x8 x = r.fx[j][tm];
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = f2bf(__fmul_rn(__fmul_rn(bf2f(x[e]), rs[tm]), bf2f(gv[e])));
@@ -517,7 +526,7 @@ __device__ void gemm_epilogue(CPhase& P, const EpiItem& it, const EpiPre& e,
   if (!it.on) return;
   const int m = it.ml, n = it.n;
   auto get = [&](int nl, float v[4]) {
-    const f32x4 t = sum_parts(sh, m, nl);
+    const f32x4 t = sum_parts(sh, it.pr, nl);
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = t[i];
   };
@@ -588,9 +597,10 @@ __device__ void gemm_epilogue(CPhase& P, const EpiItem& it, const EpiPre& e,
 }
 
 // one V^T word: item = (sample b, key quad kq, tile column c)
-__device__ __forceinline__ void vt_item(CPhase& P, int ct, const XShared& sh, int item) {
+__device__ __forceinline__ void vt_item(CPhase& P, int cg, int ct, int t0, const XShared& sh,
+                                        int item) {
   const int c = item & 15, kq = (item >> 4) & 15, b = item >> 8;
-  const int base = tile_base(P.epi, ct);
+  const int base = tile_base(P.epi, cg * P.cts + ct);
   const int col = (c < 8 ? base + c : base + 32 + (c - 8)) - P.rope_cols;
   float v[4];
 #pragma unroll
@@ -598,7 +608,7 @@ __device__ __forceinline__ void vt_item(CPhase& P, int ct, const XShared& sh, in
     const int key = 4 * kq + i;
     float t = 0.f;
     if (key < P.chunk) {
-      const int ml = b * P.chunk + key;
+      const int ml = part_row(ct, b * P.chunk + key, t0);
 #pragma unroll
       for (int w = 0; w < XW; ++w) t += sh.g.part[w][ml * XPS + c];
       t = rbf(t);
@@ -614,40 +624,100 @@ __device__ __forceinline__ void vt_item(CPhase& P, int ct, const XShared& sh, in
 // V is stored as projected (no RoPE).
 // (several row groups only at one sample: key = row, so a 4-key word lies in
 // one row tile)
-__device__ void vt_epilogue(CPhase& P, int ct, const XShared& sh, int t0, int t1) {
+__device__ void vt_epilogue(CPhase& P, int cg, const XShared& sh, int t0, int t1) {
   const int nb = P.M / P.chunk;
-  for (int item = tidx(); item < 256 * nb; item += XT) {
+  for (int i = tidx(); i < 256 * nb * P.cts; i += XT) {
+    const int ct = i / (256 * nb), item = i - ct * 256 * nb;
     const int tile = ((item >> 4) & 15) >> 2;  // row tile of key 4 kq at sample 0
     if (P.row_groups > 1 && (tile < t0 || tile >= t1)) continue;
-    vt_item(P, ct, sh, item);
+    vt_item(P, cg, ct, t0, sh, item);
   }
 }
 
 
-__device__ __forceinline__ void gemm_mma(CPhase& P, const GemmRegs& r, const bf16* sw,
-                                         f32x4 (&acc)[4], int t0, int t1) {
+template <int NT, int CT>
+__device__ __forceinline__ void gemm_mma(CPhase& P, const GemmRegs<NT>& r, const bf16* sw,
+                                         f32x4 (&acc)[CT][NT]) {
   const int lane = tidx() & 63, wave = wave_id();
   const int fr = lane & 15, G = lane >> 4;
   int ks0, kcnt;
   wave_krange(P.K, wave, ks0, kcnt);
 #pragma unroll
-  for (int j = 0; j < XKS; ++j) {
+  for (int j = 0; j < XKS / CT; ++j) {
     if (j >= kcnt) break;  // wave-uniform
-    const bf16x8 fw = *reinterpret_cast<const bf16x8*>(sw + j * XWSTEP + fr * 32 + wswz(fr, G) * 8);
 #pragma unroll
-    for (int tm = 0; tm < 4; ++tm)
-      if (tm >= t0 && tm < t1)  // wave-uniform
-        acc[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw, r.fx[j][tm], acc[tm], 0, 0, 0);
+    for (int c = 0; c < CT; ++c) {
+      const bf16x8 fw = *reinterpret_cast<const bf16x8*>(sw + (c * kcnt + j) * XWSTEP + fr * 32 + wswz(fr, G) * 8);
+#pragma unroll
+      for (int tm = 0; tm < NT; ++tm)
+        acc[c][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw, r.fx[j][tm], acc[c][tm], 0, 0, 0);
+    }
   }
 }
 
-// partial tile of this wave: element (row tm*16 + fr, columns 4*(lane/16) .. +3)
-__device__ __forceinline__ void put_partial(const f32x4 (&acc)[4], XShared& sh) {
+// partial tiles of this wave: element (row tm*16 + fr, columns 4*(lane/16) .. +3)
+template <int NT, int CT>
+__device__ __forceinline__ void put_partial(const f32x4 (&acc)[CT][NT], XShared& sh) {
   const int lane = tidx() & 63, wave = wave_id();
   const int fr = lane & 15;
 #pragma unroll
-  for (int tm = 0; tm < 4; ++tm)
-    *reinterpret_cast<f32x4*>(&sh.g.part[wave][(tm * 16 + fr) * XPS + 4 * (lane >> 4)]) = acc[tm];
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int tm = 0; tm < NT; ++tm)
+      *reinterpret_cast<f32x4*>(
+          &sh.g.part[wave][part_row(c, tm * 16 + fr, 0) * XPS + 4 * (lane >> 4)]) = acc[c][tm];
+}
+
+// This workgroup's units rank, rank + team, ... of a GEMM phase (`mine` of
+// them; the first one's weights and gains were requested before the wait).
+template <int NT, int CT>
+__device__ __forceinline__ void gemm_units(CPhase& P, XShared& sh, bf16* sw, int rank, int team,
+                                           int mine) {
+  const int lane = tidx() & 63, wave = wave_id();
+  GemmRegs<NT> r;
+  for (int j = 0; j < mine; ++j) {
+    const int u = rank + j * team;
+    const int cg = u % P.col_tiles, grp = u / P.col_tiles;
+    const int t0 = grp * P.group_tiles, t1 = min(t0 + P.group_tiles, 4);
+    const bool vt = vt_unit(P, cg);
+    const EpiItem it = epi_item(P, cg, t0, t1);
+    EpiPre e{};
+    if (!vt) epi_prefetch(P, it, e);
+    // one row group: the activations stay in registers for the phase's units
+    if (j == 0 || P.row_groups > 1) {
+      load_x<NT>(P, r, t0);
+      if (P.norm_w) {
+        // per-row sums of squares of the whole K range meet in LDS, then
+        // every wave normalises its activation fragments
+#pragma unroll
+        for (int tm = 0; tm < NT; ++tm) {
+          float t = r.ss[tm];
+          t = xor32_sum(xor16_sum(t));
+          if (lane < 16) sh.g.ss[wave][(t0 + tm) * 16 + lane] = t;
+        }
+        wg_sync_lds();
+        norm_x<NT>(P, r, sh, t0);
+      }
+    }
+    f32x4 acc[CT][NT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int tm = 0; tm < NT; ++tm) acc[c][tm] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // this wave's weight DMA (issued first) and activations have landed
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(wc_vm(0));
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    gemm_mma<NT, CT>(P, r, sw, acc);
+    put_partial<NT, CT>(acc, sh);
+    wg_sync_lds();  // also: this wave's weight reads are done
+    // the next unit's weights stream in during this unit's epilogue
+    if (j + 1 < mine)
+      dma_w(P.epi, P.w, P.N, P.K, P.ldw, P.cts, (u + team) % P.col_tiles, sw);
+    if (vt) vt_epilogue(P, cg, sh, t0, t1);
+    else gemm_epilogue(P, it, e, sh);
+    wg_sync_lds();  // partial tiles free for the next unit
+  }
 }
 
 // ---- attention units -----------------------------------------------------------
@@ -1097,12 +1167,11 @@ __global__ __launch_bounds__(XT, 1) void expert_kernel(XArgs g) {
     if (rank >= P.units) continue;
     const int tid = tidx(), lane = tid & 63;  // (not hoisted: see tidx)
     const int mine = (P.units - rank + team - 1) / team;
-    GemmRegs r;
     bf16* sw = s_w[wave];
     // weights of the first unit (and the K / V^T of a cross-attention unit)
     // before the wait: they do not depend on it
     if (P.kind == XK_GEMM) {
-      dma_w(P.epi, P.w, P.N, P.K, P.ldw, rank % P.col_tiles, sw);
+      dma_w(P.epi, P.w, P.N, P.K, P.ldw, P.cts, rank % P.col_tiles, sw);
       if (P.norm_w) dma_gain(P.norm_w, P.K, sh.g.gain[wave]);
     }
     else if (P.kind == XK_ATTN && P.kv_static)
@@ -1126,47 +1195,13 @@ __global__ __launch_bounds__(XT, 1) void expert_kernel(XArgs g) {
     }
     if (g.stamps && rank == 0 && tidx() == 0) g.stamps[2 * p] = __builtin_amdgcn_s_memrealtime();
     if (P.kind == XK_GEMM) {
-      for (int j = 0; j < mine; ++j) {
-        const int u = rank + j * team;
-        const int ct = u % P.col_tiles, grp = u / P.col_tiles;
-        const int t0 = grp * P.group_tiles, t1 = min(t0 + P.group_tiles, 4);
-        const bool vt = vt_unit(P, ct);
-        const EpiItem it = epi_item(P, ct, t0, t1);
-        EpiPre e{};
-        if (!vt) epi_prefetch(P, it, e);
-        // one row group: the activations stay in registers for the phase's units
-        const bool load = j == 0 || P.row_groups > 1;
-        if (load) {
-          load_x(P, r, t0, t1);
-          if (P.norm_w) {
-            // per-row sums of squares of the whole K range meet in LDS, then
-            // every wave normalises its activation fragments
-#pragma unroll
-            for (int tm = 0; tm < 4; ++tm) {
-              float t = r.ss[tm];
-              t = xor32_sum(xor16_sum(t));
-              if (lane < 16) sh.g.ss[wave][tm * 16 + lane] = t;
-            }
-            wg_sync_lds();
-            norm_x(P, r, sh, t0, t1);
-          }
-        }
-        f32x4 acc[4];
-#pragma unroll
-        for (int tm = 0; tm < 4; ++tm) acc[tm] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // this wave's weight DMA (issued first) and activations have landed
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_s_waitcnt(wc_vm(0));
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        gemm_mma(P, r, sw, acc, t0, t1);
-        put_partial(acc, sh);
-        wg_sync_lds();  // also: this wave's weight reads are done
-        // the next unit's weights stream in during this unit's epilogue
-        if (j + 1 < mine)
-          dma_w(P.epi, P.w, P.N, P.K, P.ldw, (u + team) % P.col_tiles, sw);
-        if (vt) vt_epilogue(P, ct, sh, t0, t1);
-        else gemm_epilogue(P, it, e, sh);
-        wg_sync_lds();  // partial tiles free for the next unit
+      if (P.cts == 2) {
+        if (P.group_tiles == 2) gemm_units<2, 2>(P, sh, sw, rank, team, mine);
+        else gemm_units<1, 2>(P, sh, sw, rank, team, mine);
+      } else {
+        if (P.group_tiles == 1) gemm_units<1, 1>(P, sh, sw, rank, team, mine);
+        else if (P.group_tiles == 2) gemm_units<2, 1>(P, sh, sw, rank, team, mine);
+        else gemm_units<4, 1>(P, sh, sw, rank, team, mine);
       }
     } else if (P.kind == XK_ATTN) {
       for (int j = 0; j < mine; ++j) {
@@ -1271,6 +1306,7 @@ size_t build(const svla_expert_desc* d, char* base, std::vector<XPhase>* out, La
     P.epi = XE_STORE;
     P.M = M; P.N = N; P.K = K;
     P.col_tiles = (N + XBN - 1) / XBN;
+    P.cts = 1;
     P.units = P.col_tiles;
     P.a = a; P.lda = lda;
     P.w = static_cast<const bf16*>(w); P.ldw = K;
@@ -1399,10 +1435,26 @@ size_t build(const svla_expert_desc* d, char* base, std::vector<XPhase>* out, La
   const int nrt = (M + 15) / 16;
   for (XPhase& P : ph) {
     if (P.kind != XK_GEMM) continue;
-    int rg = 1;
-    while (rg * 2 <= nrt && P.col_tiles * rg * 2 <= kUnitTarget && (!P.vt || d->batch == 1)) rg *= 2;
+    auto groups = [&](int col_groups) {
+      int rg = 1;
+      while (rg * 2 <= nrt && col_groups * rg * 2 <= kUnitTarget && (!P.vt || d->batch == 1)) rg *= 2;
+      return rg;
+    };
+    int rg = groups(P.col_tiles);
+    // Two column tiles per unit where that halves the rows it reads: the
+    // weights stream in before the wait, the activations and their
+    // normalisation are on the critical path (norm + gate|up: 64 rows x 16
+    // columns 8.8 us, 32 x 32 PLACEHOLDER).
+    if (P.col_tiles % 2 == 0 && (P.K + 31) / 32 <= XW * XKS / 2 && (!P.vt || P.rope_cols % 32 == 0)) {
+      const int rg2 = groups(P.col_tiles / 2);
+      if (rg2 > rg && (nrt + rg2 - 1) / rg2 <= 2) {
+        rg = rg2;
+        P.cts = 2;
+        P.col_tiles /= 2;
+      }
+    }
     P.row_groups = rg;
-    P.group_tiles = rg == 1 ? 4 : (nrt + rg - 1) / rg;
+    P.group_tiles = rg == 1 ? 4 : (nrt + rg - 1) / rg;  // 4, 2 or 1 (nrt <= 4)
     P.units = P.col_tiles * rg;
   }
   L.total = ar.off;
