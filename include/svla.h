@@ -365,7 +365,7 @@ typedef struct svla_expert_plan {
 
 /* Device workspace bytes svla_expert_prepare needs for d (phase table,
  * arrival counters, and one buffer per intermediate activation of the whole
- * chunk: about 9.4 MB per Euler step at batch 1), or 0 if d is invalid
+ * chunk: about 11 MB per Euler step at batch 1), or 0 if d is invalid
  * (chunk > 64, head_dim != 64, hidden / inter / q width > 2048, prefix_len >
  * 256, a NULL pointer). */
 long svla_expert_workspace_size(const svla_expert_desc* d);

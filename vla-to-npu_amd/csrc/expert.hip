@@ -17,12 +17,15 @@
 //    attention); unit u of a phase runs on team rank u % team_size.
 //  * Phases hand over through device-scope arrival counters: a workgroup
 //    that finished its units of phase p waits for its stores to be
-//    acknowledged (vmcnt = 0), then adds its unit count to one of 8
-//    sub-counters of phase p (spread so that 256 arrivals do not queue on
-//    one address: a grid barrier measured 4.0 us with one counter, 2.0 us
-//    with 8); a workgroup with units in phase p + 1 polls the 8
-//    sub-counters (with the status word, one round trip per poll) until they
-//    sum to phase p's unit count.  Completion of phase p implies completion
+//    acknowledged (vmcnt = 0), then adds its unit count to one of 16
+//    sub-counters of phase p in each of 8 replicas (one instruction, a lane
+//    per replica); a workgroup with units in phase p + 1 polls the
+//    sub-counters of replica rank % 8 (with the status word, one round trip
+//    per poll) until they sum to phase p's unit count.  Arrivals queue behind
+//    each other and behind the polls of one address, so both are spread: with
+//    8 unreplicated sub-counters, all polled by up to 256 workgroups, the
+//    launch took 4.75 ms, with 16 4.56, with 8 replicas of 8 4.26, of 16
+//    4.23 (4 sub-counters: 5.08).  Completion of phase p implies completion
 //    of every earlier phase (each of its units waited for p - 1), so one
 //    wait per phase suffices.
 //  * Every phase writes its output to a buffer that no other phase of the
@@ -85,7 +88,8 @@ constexpr int XKW = 64;            // attention: keys of the one-wave-per-query-
 constexpr int XKG = XMAXK / XW;    // attention: keys per wave of the split path (32)
 constexpr int XVTS = 64;           // self-attention V^T: keys per sample (leading dimension)
 constexpr int kMaxCross = 16;      // cross layers (V^T transposes in the first phase)
-constexpr int kSub = 8;            // sub-counters per phase
+constexpr int kSub = 16;           // sub-counters per phase and replica
+constexpr int kRep = 8;            // counter replicas: one for every kRep-th workgroup
 constexpr int kCntStride = 32;     // unsigned per sub-counter (128 bytes apart)
 constexpr int kSpin = 1 << 22;     // polls before a wait gives up
 
@@ -216,18 +220,20 @@ __device__ __forceinline__ void st2f_wt(float* p, float a, float b) {
                                                __builtin_bit_cast(uint32_t, b)}));
 }
 
-// Wave 0 polls the 8 sub-counters of `row` (lanes 0..7) and the status word
-// (lane 8) together until the counters sum to `target`; false when the wait
-// gave up (status set).
-__device__ bool wait_phase(const XArgs& g, int row, unsigned target) {
+__device__ __forceinline__ unsigned* sub_counter(const XArgs& g, int row, int rep, int sub) {
+  return g.cnt + (((size_t)row * kRep + rep) * kSub + sub) * kCntStride;
+}
+// Wave 0 polls the sub-counters of `row` in replica `rep` (lanes 0..kSub-1)
+// and the status word (lane kSub) together until the counters sum to
+// `target`; false when the wait gave up (status set).
+__device__ bool wait_phase(const XArgs& g, int row, int rep, unsigned target) {
   const int lane = tidx() & 63;
-  const unsigned* c = lane < kSub ? g.cnt + ((size_t)row * kSub + lane) * kCntStride : g.status;
+  const unsigned* c = lane < kSub ? sub_counter(g, row, rep, lane) : g.status;
   for (int n = 0;; ++n) {
     const unsigned v = lane <= kSub ? ld_agent(c) : 0u;
     unsigned s = lane < kSub ? v : 0u;
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    s += __shfl_xor(s, 4, 64);
+#pragma unroll
+    for (int o = 1; o < kSub; o <<= 1) s += __shfl_xor(s, o, 64);
     const unsigned st = __shfl(v, kSub, 64);
     if (__builtin_amdgcn_readfirstlane(s) >= target) return true;
     if (__builtin_amdgcn_readfirstlane(st) != 0u) return false;
@@ -1094,7 +1100,7 @@ __device__ void poison_actions(const XArgs& g) {
 __device__ void team_watch(const XArgs& g) {
   __shared__ int s_fail;
   if (wave_id() == 0) {
-    const unsigned* reg = g.cnt + (size_t)g.n_ph * kSub * kCntStride;
+    const unsigned* reg = g.cnt + (size_t)g.n_ph * kRep * kSub * kCntStride;
     bool fail = true;
     for (int n = 0; n < g.spin; ++n) {
       if (__builtin_amdgcn_readfirstlane(ld_agent(reg)) >= (unsigned)g.team_size ||
@@ -1124,7 +1130,7 @@ __global__ __launch_bounds__(XT, 1) void expert_kernel(XArgs g) {
       asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(x));
       rank = -1;
       if ((int)(x & 15u) == g.team_xcd) {
-        unsigned* reg = g.cnt + (size_t)g.n_ph * kSub * kCntStride;
+        unsigned* reg = g.cnt + (size_t)g.n_ph * kRep * kSub * kCntStride;
         const unsigned r =
             __hip_atomic_fetch_add(reg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         rank = r < (unsigned)g.team_size ? (int)r : -1;
@@ -1143,7 +1149,7 @@ __global__ __launch_bounds__(XT, 1) void expert_kernel(XArgs g) {
   if (g.team_xcd >= 0) {
     if (wave == 0) {
       // every member registered before anyone relies on the team's size
-      const unsigned* reg = g.cnt + (size_t)g.n_ph * kSub * kCntStride;
+      const unsigned* reg = g.cnt + (size_t)g.n_ph * kRep * kSub * kCntStride;
       bool ok = false;
       for (int n = 0; n < g.spin; ++n) {
         const unsigned rr = __builtin_amdgcn_readfirstlane(ld_agent(reg));
@@ -1184,7 +1190,7 @@ __global__ __launch_bounds__(XT, 1) void expert_kernel(XArgs g) {
         asm volatile("" ::"s"(t));
       }
       if (wave == 0) {
-        const bool ok = wait_phase(g, p - 1, (unsigned)g.ph[p - 1].units);
+        const bool ok = wait_phase(g, p - 1, rank % kRep, (unsigned)g.ph[p - 1].units);
         if (lane == 0) s_rank = ok ? rank : -1;
       }
       __syncthreads();
@@ -1214,11 +1220,10 @@ __global__ __launch_bounds__(XT, 1) void expert_kernel(XArgs g) {
     // every store of this workgroup acknowledged, then one arrival
     __builtin_amdgcn_s_waitcnt(wc_vm(0));
     __syncthreads();
-    if (tid == 0) {
-      __hip_atomic_fetch_add(g.cnt + ((size_t)p * kSub + (rank & (kSub - 1))) * kCntStride,
-                             (unsigned)mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (g.stamps && rank == 0) g.stamps[2 * p + 1] = __builtin_amdgcn_s_memrealtime();
-    }
+    if (tid < kRep)  // one instruction: a lane per replica
+      __hip_atomic_fetch_add(sub_counter(g, p, tid, rank / kRep % kSub), (unsigned)mine,
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (g.stamps && rank == 0 && tid == 0) g.stamps[2 * p + 1] = __builtin_amdgcn_s_memrealtime();
   }
   if (failed) poison_actions(g);
 }
@@ -1287,7 +1292,7 @@ size_t build(const svla_expert_desc* d, char* base, std::vector<XPhase>* out, La
             kvd = d->n_kv_heads * 64, I = d->inter, A = d->action_dim;
   Layout L{};
   L.n_ph = count_phases(d);
-  L.n_cnt_words = (size_t)(L.n_ph + 1) * kSub * kCntStride;
+  L.n_cnt_words = (size_t)(L.n_ph + 1) * kRep * kSub * kCntStride;
   Arena ar;
   L.phases = ar.take(sizeof(XPhase) * L.n_ph);
   L.counters = ar.take(L.n_cnt_words * 4);
@@ -1443,8 +1448,8 @@ size_t build(const svla_expert_desc* d, char* base, std::vector<XPhase>* out, La
     int rg = groups(P.col_tiles);
     // Two column tiles per unit where that halves the rows it reads: the
     // weights stream in before the wait, the activations and their
-    // normalisation are on the critical path (norm + gate|up: 64 rows x 16
-    // columns 8.8 us, 32 x 32 PLACEHOLDER).
+    // normalisation are on the critical path (norm + gate|up with its
+    // run-time unit bounds: 64 rows x 16 columns 8.8 us, 32 x 32 7.9).
     if (P.col_tiles % 2 == 0 && (P.K + 31) / 32 <= XW * XKS / 2 && (!P.vt || P.rope_cols % 32 == 0)) {
       const int rg2 = groups(P.col_tiles / 2);
       if (rg2 > rg && (nrt + rg2 - 1) / rg2 <= 2) {
