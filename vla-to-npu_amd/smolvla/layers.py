@@ -210,11 +210,13 @@ def _normed(x, w, eps, M, bufs, name):
 
 
 def decoder_layer(x, P, cfg: DecoderConfig, B, L, rope: Rope, mask="causal", prefix_len=0,
-                  bufs: Optional[Buffers] = None, qkv_out=None, mid_out=None):
-    """One SmolLM2-style block on ``x [B*L, H]`` **in place**; returns the
-    fused projection buffer ``[B*L, q|k|v]`` whose K (post-RoPE) and V column
-    slices are this layer's KV cache (vla/text_encoder_bf16.py:480-595).
-    ``mid_out`` (optional) receives the mid-block residual (after attention)."""
+                  bufs: Optional[Buffers] = None, qkv_out=None, mid_out=None, out=None):
+    """One SmolLM2-style block on ``x [B*L, H]``, **in place** or into ``out``
+    (``x`` is then only read); returns the fused projection buffer
+    ``[B*L, q|k|v]`` whose K (post-RoPE) and V column slices are this layer's
+    KV cache (vla/text_encoder_bf16.py:480-595).  ``mid_out`` (optional)
+    receives the mid-block residual (after attention)."""
+    out = x if out is None else out
     bufs = bufs or Buffers(x.device)
     M = B * L
     qd, kvd = cfg.q_dim, cfg.kv_dim
@@ -231,10 +233,10 @@ def decoder_layer(x, P, cfg: DecoderConfig, B, L, rope: Rope, mask="causal", pre
     ops.attention(q3[:, :, :qd], q3[:, :, qd:qd + kvd], q3[:, :, qd + kvd:],
                   attn.view(B, L, qd), cfg.n_q_heads, cfg.n_kv_heads, mask, prefix_len,
                   q_lo=l3[:, :, :qd], k_lo=l3[:, :, qd:qd + kvd])
-    ops.linear(attn, P["wo"], res=x, out=x)
+    ops.linear(attn, P["wo"], res=x, out=out)
     if mid_out is not None:
-        mid_out.copy_(x)
-    _mlp(x, P, cfg, M, eps, bufs)
+        mid_out.copy_(out)
+    _mlp(out, P, cfg, M, eps, bufs)
     return qkv
 
 
@@ -273,10 +275,11 @@ def cross_kv(k_src, v_src, P, out_k=None, out_v=None):
 
 
 def cross_layer(x, ck, cv, P, cfg: DecoderConfig, B, L, Lc, rope: Rope,
-                bufs: Optional[Buffers] = None):
-    """Expert cross-attention block on ``x [B*L, H]`` in place, attending to
-    the already projected ``ck``/``cv [B*Lc, kv]`` (vla/action_expert_bf16.py:731-803;
+                bufs: Optional[Buffers] = None, out=None):
+    """Expert cross-attention block on ``x [B*L, H]``, in place or into ``out``,
+    attending to the already projected ``ck``/``cv [B*Lc, kv]`` (vla/action_expert_bf16.py:731-803;
     RoPE on Q only, no mask)."""
+    out = x if out is None else out
     bufs = bufs or Buffers(x.device)
     M = B * L
     qd = cfg.q_dim
@@ -288,12 +291,13 @@ def cross_layer(x, ck, cv, P, cfg: DecoderConfig, B, L, Lc, rope: Rope,
     attn = bufs.get("attn", M, qd)
     ops.attention(q.view(B, L, qd), ck.view(B, Lc, -1), cv.view(B, Lc, -1), attn.view(B, L, qd),
                   cfg.n_q_heads, cfg.n_kv_heads, "none", 0, q_lo=q_lo.view(B, L, qd))
-    ops.linear(attn, P["wo"], res=x, out=x)
-    _mlp(x, P, cfg, M, eps, bufs)
+    ops.linear(attn, P["wo"], res=x, out=out)
+    _mlp(out, P, cfg, M, eps, bufs)
 
 
-def vit_layer(x, P, cfg: VitConfig, n_img, T, bufs: Optional[Buffers] = None, plan=None):
-    """SigLIP-style block on ``x [n_img*T, H]`` in place
+def vit_layer(x, P, cfg: VitConfig, n_img, T, bufs: Optional[Buffers] = None, plan=None,
+              out=None):
+    """SigLIP-style block on ``x [n_img*T, H]``, in place or into ``out``
     (vla/vision_block_bf16.py:308-420).  Each projection that ``plan``
     (default: :func:`vit_blocked_plan` at these rows) marks and whose
     slab-blocked weight ``P`` holds runs on the 256x256 GEMM, and the
@@ -301,19 +305,20 @@ def vit_layer(x, P, cfg: VitConfig, n_img, T, bufs: Optional[Buffers] = None, pl
     its K loop streams both operands as contiguous kilobytes; the others run
     on the automatic tile choice.  The residual stream stays row-major."""
     from .ops import LAYOUT_A_BLOCKED as AB, LAYOUT_W_BLOCKED as WB, LAYOUT_C_BLOCKED as CB
+    y = x if out is None else out        # the residual stream after attention
     bufs = bufs or Buffers(x.device)
     M, H, I = n_img * T, cfg.hidden, cfg.inter
     plan = plan or vit_blocked_plan(H, I, M)
     blk = {k: bool(plan[k]) and w + "_blk" in P for k, w in VIT_PROJ.items()}
     blk["down"] = blk["down"] and blk["up"]
 
-    def norm(g, b, blocked):
-        out = bufs.get("vh", M, H)
+    def norm(t, g, b, blocked):
+        h = bufs.get("vh", M, H)
         if blocked:
-            return ops.layernorm(x, g, b, cfg.ln_eps, out=out.view(H // 32, M, 32), blocked=True)
-        return ops.layernorm(x, g, b, cfg.ln_eps, out=out)
+            return ops.layernorm(t, g, b, cfg.ln_eps, out=h.view(H // 32, M, 32), blocked=True)
+        return ops.layernorm(t, g, b, cfg.ln_eps, out=h)
 
-    h = norm(P["g1"], P["b1"], blk["qkv"])
+    h = norm(x, P["g1"], P["b1"], blk["qkv"])
     qkv = bufs.get("vqkv", M, 3 * H)
     if blk["qkv"]:
         ops.linear_wide(h, P["wqkv_blk"], M, 3 * H, H, bias=P["bqkv"], out=qkv, layout=AB | WB)
@@ -324,21 +329,21 @@ def vit_layer(x, P, cfg: VitConfig, n_img, T, bufs: Optional[Buffers] = None, pl
     ops.attention(q3[:, :, :H], q3[:, :, H:2 * H], q3[:, :, 2 * H:], attn.view(n_img, T, H),
                   cfg.n_heads, cfg.n_heads, "none", 0, scale=1.0 / math.sqrt(cfg.head_dim))
     if blk["o"]:
-        ops.linear_wide(attn, P["wo_blk"], M, H, H, bias=P["bo"], res=x, out=x, layout=WB)
+        ops.linear_wide(attn, P["wo_blk"], M, H, H, bias=P["bo"], res=x, out=y, layout=WB)
     else:
-        ops.linear(attn, P["wo"], bias=P["bo"], res=x, out=x)
-    h = norm(P["g2"], P["b2"], blk["up"])
+        ops.linear(attn, P["wo"], bias=P["bo"], res=x, out=y)
+    h = norm(y, P["g2"], P["b2"], blk["up"])
     gelu = "gelu_" + cfg.gelu
     act = bufs.get("vmlp", M, I)
     if blk["down"]:                       # up is blocked too: hand the activation over blocked
         act = act.view(I // 32, M, 32)
         ops.linear_wide(h, P["wup_blk"], M, I, H, bias=P["bup"], act=gelu, out=act,
                         layout=AB | WB | CB)
-        ops.linear_wide(act, P["wd_blk"], M, H, I, bias=P["bd"], res=x, out=x, layout=AB | WB)
+        ops.linear_wide(act, P["wd_blk"], M, H, I, bias=P["bd"], res=y, out=y, layout=AB | WB)
         return
     if blk["up"]:
         ops.linear_wide(h, P["wup_blk"], M, I, H, bias=P["bup"], act=gelu, out=act,
                         layout=AB | WB)
     else:
         ops.linear(h, P["wup"], bias=P["bup"], act=gelu, out=act)
-    ops.linear(act, P["wd"], bias=P["bd"], res=x, out=x)
+    ops.linear(act, P["wd"], bias=P["bd"], res=y, out=y)

@@ -48,6 +48,13 @@ def as_batched(x):
     return x, False
 
 
+def as_rows(x3):
+    """``[B, L, H] -> [B*L, H]`` rows the kernels can read: contiguous and
+    16-byte aligned (a view of the caller's tensor where it already is)."""
+    x2 = x3.reshape(-1, x3.shape[-1]).contiguous()
+    return x2.clone() if x2.data_ptr() % 16 else x2
+
+
 # Packed weights of recently used params dicts.  Kept here, not in the
 # caller's dict: an entry is reused only while the dict holds the very same
 # weight objects with unchanged contents (torch tensors: the version counter

@@ -12,9 +12,11 @@ text encoder's K/V, no mask.  Defaults are the target expert width (hidden
 
 from __future__ import annotations
 
+import torch
+
 from .. import layers
 from ..config import DecoderConfig
-from ._common import as_batched, prepared, to_device
+from ._common import as_batched, as_rows, prepared, to_device
 
 SEQ = 50
 TEXT_SEQ = 241
@@ -32,9 +34,10 @@ def action_expert_self_forward(x_np, params, cfg: DecoderConfig = DEFAULT_CFG):
     x3, squeeze = as_batched(x)
     B, L, H = x3.shape
     P = prepared(params, layers.prep_decoder)
-    out = x3.reshape(B * L, H).clone()
+    x2 = as_rows(x3)
+    out = torch.empty_like(x2)
     rope = layers.Rope.make(L, cfg.head_dim, cfg.rope_theta, out.device)
-    layers.decoder_layer(out, P, cfg, B, L, rope, "causal", 0)
+    layers.decoder_layer(x2, P, cfg, B, L, rope, "causal", 0, out=out)
     return back(out.view(L, H) if squeeze else out.view(B, L, H))
 
 
@@ -50,7 +53,8 @@ def action_expert_cross_forward(x_np, text_k_np, text_v_np, params,
     Lc = tk3.shape[1]
     P = prepared(params, layers.prep_cross)
     ck, cv = layers.cross_kv(tk3.reshape(B * Lc, -1), tv3.reshape(B * Lc, -1), P)
-    out = x3.reshape(B * L, H).clone()
+    x2 = as_rows(x3)
+    out = torch.empty_like(x2)
     rope = layers.Rope.make(L, cfg.head_dim, cfg.rope_theta, out.device)
-    layers.cross_layer(out, ck, cv, P, cfg, B, L, Lc, rope)
+    layers.cross_layer(x2, ck, cv, P, cfg, B, L, Lc, rope, out=out)
     return back(out.view(L, H) if squeeze else out.view(B, L, H))

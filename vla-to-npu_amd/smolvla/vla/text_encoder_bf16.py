@@ -19,7 +19,7 @@ import torch
 
 from .. import layers, ops
 from ..config import DecoderConfig, resolve_eps
-from ._common import as_batched, prepared, to_device
+from ._common import as_batched, as_rows, prepared, to_device
 
 SEQ = 128
 EMBD = 960
@@ -38,13 +38,15 @@ def text_encoder_forward(x_np, params, cfg: DecoderConfig = DEFAULT_CFG, mask="c
     B, L, H = x3.shape
     P = prepared(params, layers.prep_decoder)
     qd, kvd = cfg.q_dim, cfg.kv_dim
-    out = x3.reshape(B * L, H).clone()
+    x2 = as_rows(x3)
+    out = torch.empty_like(x2)
     rope = layers.Rope.make(L, cfg.head_dim, cfg.rope_theta, out.device)
     bufs = layers.Buffers(out.device)
     mid = torch.empty_like(out) if kv_export == "torch_ref" else None
-    qkv = layers.decoder_layer(out, P, cfg, B, L, rope, mask, prefix_len, bufs, mid_out=mid)
+    qkv = layers.decoder_layer(x2, P, cfg, B, L, rope, mask, prefix_len, bufs, mid_out=mid, out=out)
     if kv_export == "cache":
-        key, value = qkv[:, qd:qd + kvd].clone(), qkv[:, qd + kvd:].clone()
+        # K and V leave the fused projection in one copy
+        key, value = qkv[:, qd:].view(B * L, 2, kvd).transpose(0, 1).contiguous().unbind(0)
     elif kv_export == "torch_ref":
         hn = ops.rmsnorm(mid, P["n1"], resolve_eps(cfg.rms_eps))
         key = ops.linear(hn, P["wqkv"][qd:qd + kvd])

@@ -10,9 +10,11 @@ module's choices are ``VitConfig(ln_eps=1e-5, gelu="erf")``.
 
 from __future__ import annotations
 
+import torch
+
 from .. import layers
 from ..config import VitConfig
-from ._common import as_batched, prepared, to_device
+from ._common import as_batched, as_rows, prepared, to_device
 
 SEQ = 1024
 EMBD = 768
@@ -22,13 +24,22 @@ FFN_HID = 3072
 DEFAULT_CFG = VitConfig()
 
 
+def _prep_blocked(p, device):
+    """Weights for calls whose rows put projections on the slab-blocked
+    256x256 GEMM: blocked copies of every projection that a large enough call
+    moves there (each call's own plan picks among them)."""
+    return layers.prep_vit(p, device, rows=1 << 20)
+
+
 def vision_block(x_np, params, cfg: VitConfig = DEFAULT_CFG):
     x, back = to_device(x_np)
     x3, squeeze = as_batched(x)
     B, T, H = x3.shape
-    P = prepared(params, layers.prep_vit)
-    out = x3.reshape(B * T, H).clone()
-    layers.vit_layer(out, P, cfg, B, T)
+    x2 = as_rows(x3)
+    plan = layers.vit_blocked_plan(H, params["W_up"].shape[1], B * T)
+    P = prepared(params, _prep_blocked if any(plan.values()) else layers.prep_vit)
+    out = torch.empty_like(x2)
+    layers.vit_layer(x2, P, cfg, B, T, out=out)
     return back(out.view(T, H) if squeeze else out.view(B, T, H))
 
 
