@@ -109,6 +109,12 @@ int svla_init(void);
 int svla_rmsnorm_bf16(const void* x, int ldx, const void* w, void* y, int ldy, int rows,
                       int cols, float eps, svla_stream_t stream);
 
+/* svla_rmsnorm_bf16 and svla_rope_table in one launch (a layer call's first
+ * norm and its tables). */
+int svla_rmsnorm_rope_table_bf16(const void* x, int ldx, const void* w, void* y, int ldy, int rows,
+                                 int cols, float eps, float* cos_t, float* sin_t, int max_pos,
+                                 int head_dim, float theta, svla_stream_t stream);
+
 /* LayerNorm with affine gamma/beta (beta may be NULL).
  * Replaces layer_norm_bf16 + the bias kernel (cc/bf16_old/layer_norm_bf16.cc:67;
  * vla/vision_block_bf16.py:101-127) and layernorm() (:272-280). */

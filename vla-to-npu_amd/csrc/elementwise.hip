@@ -135,17 +135,10 @@ __global__ void rope_kernel(const void* __restrict__ x, long ldx, void* __restri
   }
 }
 
-// angle = pos / theta^(2k/D): the timescale is formed in fp32 exactly as
-// apply_rope does (theta ** ((2/D) * k), vla/text_encoder_bf16.py:80-84).
 __global__ void rope_table_kernel(float* ct, float* st, int max_pos, int half, float theta,
                                   float two_over_d) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= max_pos * half) return;
-  const int pos = idx / half, k = idx % half;
-  const float ts = powf(theta, two_over_d * (float)k);
-  const float ang = (float)pos / ts;
-  ct[idx] = cosf(ang);
-  st[idx] = sinf(ang);
+  if (idx < max_pos * half) rope_entry(ct, st, idx, half, theta, two_over_d);
 }
 
 __global__ void transpose_kernel(const bf16* __restrict__ w, long ldw, bf16* __restrict__ o,

@@ -15,10 +15,9 @@ constexpr int MAXC = 4;  // 16-byte chunks per lane: cols <= 4 * 8 * 64 = 2048
 
 // (The GEMMs' fused norm, norm_rows in gemm.hip, reproduces this kernel's
 // sum of squares operation by operation: change both together.)
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const bf16* __restrict__ x, long ldx,
-                                                      const bf16* __restrict__ w,
-                                                      bf16* __restrict__ y, long ldy, int rows,
-                                                      int cols, float eps) {
+__device__ __forceinline__ void rmsnorm_rows(const bf16* __restrict__ x, long ldx,
+                                             const bf16* __restrict__ w, bf16* __restrict__ y,
+                                             long ldy, int rows, int cols, float eps) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -56,6 +55,33 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const bf16* __restrict__ x
       st8(yr + c, o);
     }
   }
+}
+
+__global__ __launch_bounds__(256) void rmsnorm_kernel(const bf16* __restrict__ x, long ldx,
+                                                      const bf16* __restrict__ w,
+                                                      bf16* __restrict__ y, long ldy, int rows,
+                                                      int cols, float eps) {
+  rmsnorm_rows(x, ldx, w, y, ldy, rows, cols, eps);
+}
+
+// The RMSNorm and, on the blocks past its own, the RoPE tables of the same
+// layer call: a table has a few thousand entries, so its own launch (3.0-3.5 us)
+// cost as much as the norm of a small layer.  MI355X, graph replay, two launches
+// / one: expert self layer 32x50 rows 75.6 / 72.8 us, text layer 5x333 rows
+// 104.2 / 101.4, 32x241 261.0 / 253.9, cross layer 50 rows 56.8 / 55.0.
+__global__ __launch_bounds__(256) void rmsnorm_table_kernel(const bf16* __restrict__ x, long ldx,
+                                                            const bf16* __restrict__ w,
+                                                            bf16* __restrict__ y, long ldy, int rows,
+                                                            int cols, float eps, float* ct, float* st,
+                                                            int entries, int half, float theta,
+                                                            float two_over_d) {
+  const int nb = (rows + 3) / 4;
+  if ((int)blockIdx.x < nb) {
+    rmsnorm_rows(x, ldx, w, y, ldy, rows, cols, eps);
+    return;
+  }
+  const int idx = ((int)blockIdx.x - nb) * 256 + threadIdx.x;
+  if (idx < entries) rope_entry(ct, st, idx, half, theta, two_over_d);
 }
 
 // Sum over the LPR lanes of each row group (LPR = 64: the whole wave; 32:
@@ -168,6 +194,21 @@ extern "C" int svla_rmsnorm_bf16(const void* x, int ldx, const void* w, void* y,
   hipLaunchKernelGGL(rmsnorm_kernel, dim3((rows + 3) / 4), dim3(256), 0, (hipStream_t)stream,
                      static_cast<const bf16*>(x), (long)ldx, static_cast<const bf16*>(w),
                      static_cast<bf16*>(y), (long)ldy, rows, cols, eps);
+  SVLA_CHECK_LAUNCH();
+  return SVLA_OK;
+}
+
+extern "C" int svla_rmsnorm_rope_table_bf16(const void* x, int ldx, const void* w, void* y, int ldy,
+                                            int rows, int cols, float eps, float* cos_t,
+                                            float* sin_t, int max_pos, int head_dim, float theta,
+                                            svla_stream_t stream) {
+  if (!norm_args_ok(x, ldx, y, ldy, cols) || !svla_aligned16(w) || rows < 0) return SVLA_EINVAL;
+  if (max_pos <= 0 || head_dim <= 0 || head_dim % 2 || !cos_t || !sin_t) return SVLA_EINVAL;
+  const int half = head_dim / 2, entries = max_pos * half;
+  hipLaunchKernelGGL(rmsnorm_table_kernel, dim3((rows + 3) / 4 + (entries + 255) / 256), dim3(256), 0,
+                     (hipStream_t)stream, static_cast<const bf16*>(x), (long)ldx,
+                     static_cast<const bf16*>(w), static_cast<bf16*>(y), (long)ldy, rows, cols, eps,
+                     cos_t, sin_t, entries, half, theta, 2.0f / (float)head_dim);
   SVLA_CHECK_LAUNCH();
   return SVLA_OK;
 }

@@ -100,6 +100,18 @@ __device__ __forceinline__ float gelu_erf_f(float x) {
   return 0.5f * x * (1.0f + erff(x * 0.7071067811865476f));
 }
 
+// Entry idx = pos * half + k of the RoPE tables, angle = pos / theta^(2k/D):
+// the timescale is formed in fp32 exactly as apply_rope does
+// (theta ** ((2/D) * k), vla/text_encoder_bf16.py:80-84).
+__device__ __forceinline__ void rope_entry(float* ct, float* st, int idx, int half, float theta,
+                                           float two_over_d) {
+  const int pos = idx / half, k = idx % half;
+  const float ts = powf(theta, two_over_d * (float)k);
+  const float ang = (float)pos / ts;
+  ct[idx] = cosf(ang);
+  st[idx] = sinf(ang);
+}
+
 #define SVLA_CHECK_LAUNCH()                        \
   do {                                             \
     hipError_t e__ = hipGetLastError();            \

@@ -172,11 +172,18 @@ class Rope:
     cos: torch.Tensor
     sin: torch.Tensor
     seq_len: int
+    theta: Optional[float] = None   # set: the tables are still to be written
 
     @classmethod
     def make(cls, seq_len, head_dim, theta, device):
         c, s = ops.rope_table(seq_len, head_dim, theta, device=device)
         return cls(c, s, seq_len)
+
+    @classmethod
+    def pending(cls, seq_len, head_dim, theta, device):
+        """For one layer call: the tables are written beside its first norm."""
+        c = torch.empty(seq_len, head_dim // 2, dtype=torch.float32, device=device)
+        return cls(c, torch.empty_like(c), seq_len, theta)
 
 
 class Buffers:
@@ -200,10 +207,15 @@ class Buffers:
 FUSED_NORM_MAX_ROWS = 0
 
 
-def _normed(x, w, eps, M, bufs, name):
+def _normed(x, w, eps, M, bufs, name, rope=None):
     """(A operand, norm argument) for a GEMM that consumes RMSNorm(x): fused
     into the GEMM up to FUSED_NORM_MAX_ROWS rows, else a standalone RMSNorm
-    into a buffer."""
+    into a buffer.  Pending tables of ``rope`` are written on the way."""
+    theta = rope.theta if rope is not None else None
+    if theta is not None:
+        rope.theta = None
+        out = bufs.get(name, M, x.shape[1])
+        return ops.rmsnorm_rope_table(x, w, eps, rope.cos, rope.sin, theta, out=out), None
     if M <= FUSED_NORM_MAX_ROWS:
         return x, (w, eps)
     return ops.rmsnorm(x, w, eps, out=bufs.get(name, M, x.shape[1])), None
@@ -226,7 +238,7 @@ def decoder_layer(x, P, cfg: DecoderConfig, B, L, rope: Rope, mask="causal", pre
     # scores in fp32 (vla/text_encoder_bf16.py:92-104, 117-122); the cache
     # keeps the bf16 values (:595)
     lo = bufs.get("qkv_lo", M, qkv.stride(0))[:, :qd + 2 * kvd]
-    a, nrm = _normed(x, P["n1"], eps, M, bufs, "xn")
+    a, nrm = _normed(x, P["n1"], eps, M, bufs, "xn", rope)
     ops.linear_rope(a, P["wqkv"], qd + kvd, L, rope.cos, rope.sin, out=qkv, norm=nrm, out_lo=lo)
     q3, l3 = qkv.view(B, L, -1), lo.view(B, L, -1)
     attn = bufs.get("attn", M, qd)
@@ -284,7 +296,7 @@ def cross_layer(x, ck, cv, P, cfg: DecoderConfig, B, L, Lc, rope: Rope,
     M = B * L
     qd = cfg.q_dim
     eps = resolve_eps(cfg.rms_eps)
-    a, nrm = _normed(x, P["n1"], eps, M, bufs, "xn")
+    a, nrm = _normed(x, P["n1"], eps, M, bufs, "xn", rope)
     q_lo = bufs.get("q_lo", M, qd)
     q = ops.linear_rope(a, P["wq"], qd, L, rope.cos, rope.sin, out=bufs.get("q", M, qd),
                         norm=nrm, out_lo=q_lo)

@@ -69,6 +69,18 @@ def rmsnorm(x, w, eps, out=None):
     return out
 
 
+def rmsnorm_rope_table(x, w, eps, cos_t, sin_t, theta, out=None):
+    """:func:`rmsnorm` and, into ``cos_t`` / ``sin_t`` ``[L, D/2]``,
+    :func:`rope_table` in one launch."""
+    eps = torch.finfo(F32).eps if eps is None else eps
+    rows, cols = x.shape
+    out = torch.empty(rows, cols, dtype=BF16, device=x.device) if out is None else out
+    _lib.call("svla_rmsnorm_rope_table_bf16", _ptr(x), _ld(x), _ptr(w), _ptr(out), _ld(out), rows,
+              cols, float(eps), _ptr(cos_t), _ptr(sin_t), cos_t.shape[0], 2 * cos_t.shape[1],
+              float(theta), _stream())
+    return out
+
+
 def layernorm(x, g, b, eps, out=None, blocked=False):
     """LayerNorm of the rows of ``x``; ``blocked`` writes the slab-blocked
     ``[cols/32, rows, 32]`` layout (``LAYOUT_A_BLOCKED`` of :func:`linear_wide`)."""

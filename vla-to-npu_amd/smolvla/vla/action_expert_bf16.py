@@ -36,7 +36,7 @@ def action_expert_self_forward(x_np, params, cfg: DecoderConfig = DEFAULT_CFG):
     P = prepared(params, layers.prep_decoder)
     x2 = as_rows(x3)
     out = torch.empty_like(x2)
-    rope = layers.Rope.make(L, cfg.head_dim, cfg.rope_theta, out.device)
+    rope = layers.Rope.pending(L, cfg.head_dim, cfg.rope_theta, out.device)
     layers.decoder_layer(x2, P, cfg, B, L, rope, "causal", 0, out=out)
     return back(out.view(L, H) if squeeze else out.view(B, L, H))
 
@@ -55,6 +55,6 @@ def action_expert_cross_forward(x_np, text_k_np, text_v_np, params,
     ck, cv = layers.cross_kv(tk3.reshape(B * Lc, -1), tv3.reshape(B * Lc, -1), P)
     x2 = as_rows(x3)
     out = torch.empty_like(x2)
-    rope = layers.Rope.make(L, cfg.head_dim, cfg.rope_theta, out.device)
+    rope = layers.Rope.pending(L, cfg.head_dim, cfg.rope_theta, out.device)
     layers.cross_layer(x2, ck, cv, P, cfg, B, L, Lc, rope, out=out)
     return back(out.view(L, H) if squeeze else out.view(B, L, H))

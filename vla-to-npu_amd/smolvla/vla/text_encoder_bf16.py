@@ -40,7 +40,7 @@ def text_encoder_forward(x_np, params, cfg: DecoderConfig = DEFAULT_CFG, mask="c
     qd, kvd = cfg.q_dim, cfg.kv_dim
     x2 = as_rows(x3)
     out = torch.empty_like(x2)
-    rope = layers.Rope.make(L, cfg.head_dim, cfg.rope_theta, out.device)
+    rope = layers.Rope.pending(L, cfg.head_dim, cfg.rope_theta, out.device)
     bufs = layers.Buffers(out.device)
     mid = torch.empty_like(out) if kv_export == "torch_ref" else None
     qkv = layers.decoder_layer(x2, P, cfg, B, L, rope, mask, prefix_len, bufs, mid_out=mid, out=out)
