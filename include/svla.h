@@ -178,6 +178,14 @@ int svla_linear_scratch_bf16(const void* a, int lda, const void* w, int ldw, con
                              int m, int n, int k, float alpha, int act, int out_f32,
                              const void* norm_w, float norm_eps, svla_stream_t stream);
 
+/* Two plain products of one shape, C0 = A0 . W0^T and C1 = A1 . W1^T (m, n, k
+ * and the leading dimensions are shared; every operand 16-byte aligned): a
+ * cross layer's K and V projections.  One launch where one product leaves most
+ * of the chip idle, else two; bit-identical to two svla_linear_bf16 calls. */
+int svla_linear_pair_bf16(const void* a0, const void* a1, int lda, const void* w0, const void* w1,
+                          int ldw, void* c0, void* c1, int ldc, int m, int n, int k,
+                          svla_stream_t stream);
+
 /* The big-problem GEMM of svla_linear_bf16 (persistent 256x256 tiles, plain
  * store epilogue: bias, fp32 bias, alpha, activation, residual) with optional
  * slab-blocked layouts (SVLA_LAYOUT_*): a slab-blocked operand streams into

@@ -960,6 +960,11 @@ constexpr int SNS = 4;  // ring stages
 
 template <int BM, int BN, int AMODE, bool NORM, int EPI, int ACT>
 __global__ __launch_bounds__(256, (BM * BN <= 2048 ? 2 : 1)) void gemm_small_kernel(GemmArgs p) {
+  if (gridDim.z > 1 && blockIdx.z) {  // uniform
+    p.a = p.a2;
+    p.b = p.b2;
+    p.c = p.c2;
+  }
   constexpr int TM = BM / 32;          // 16-row MFMA tiles per wave
   constexpr int TN = BN / 16;          // 16-column MFMA tiles per wave
   constexpr int A_DMA = BM / 32;       // 1 KB (8-row) DMA blocks per wave per stage
@@ -2489,6 +2494,31 @@ int svla_linear_bf16(const void* a, int lda, const void* w, int ldw, const void*
   p.norm_w = static_cast<const bf16*>(norm_w);
   p.norm_eps = norm_eps;
   return run_gemm<A_DENSE>(p, EPI_STORE, act, (hipStream_t)stream);
+}
+
+int svla_linear_pair_bf16(const void* a0, const void* a1, int lda, const void* w0, const void* w1,
+                          int ldw, void* c0, void* c1, int ldc, int m, int n, int k,
+                          svla_stream_t stream) {
+  GemmArgs p = base_args(a0, lda, w0, ldw, c0, ldc, m, n, k);
+  GemmArgs q = base_args(a1, lda, w1, ldw, c1, ldc, m, n, k);
+  const bool ok = m > 0 && n > 0 && k > 0 && k % 8 == 0 && n % 4 == 0 && lda % 8 == 0 &&
+                  ldw % 8 == 0 && ldc % 4 == 0 && svla_aligned16(a0) && svla_aligned16(a1) &&
+                  svla_aligned16(w0) && svla_aligned16(w1) && svla_aligned16(c0) && svla_aligned16(c1);
+  // Two launches of at most one 32x32 tile per CU each: together they are
+  // still within the two workgroups per CU up to which the small tile is
+  // chosen for one product (MI355X, graph replay, the cross layer around
+  // 241x320x320 twice, 80 tiles each: 55.0 us in two launches, 51.4 in one).
+  if (ok && g_force_tile < 0 && small_range(m, n, k, EPI_STORE) &&
+      pick_tile(m, n, k, EPI_STORE, true, n % 8 == 0 && ldc % 8 == 0, true).id == N32 &&
+      (long)((m + 31) / 32) * ((n + 31) / 32) <= kNumCU) {
+    p.a2 = q.a;
+    p.b2 = q.b;
+    p.c2 = q.c;
+    return dispatch<A_DENSE, false>(p, EPI_STORE, 0, N32, dim3((n + 31) / 32, (m + 31) / 32, 2),
+                                    (hipStream_t)stream);
+  }
+  const int rc = run_gemm<A_DENSE>(p, EPI_STORE, 0, (hipStream_t)stream);
+  return rc ? rc : run_gemm<A_DENSE>(q, EPI_STORE, 0, (hipStream_t)stream);
 }
 
 int svla_linear_scratch_bf16(const void* a, int lda, const void* w, int ldw, const void* bias,

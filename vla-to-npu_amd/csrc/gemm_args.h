@@ -61,6 +61,9 @@ struct GemmArgs {
   // so the 16 rows x 32 columns an LDS-DMA instruction fetches are one
   // contiguous kilobyte (the row-major layout gives 16 separate 64-byte pieces)
   int a_blk, b_blk, c_blk;
+  // second product of a pair (gemm_small_kernel, blockIdx.z == 1)
+  const bf16 *a2, *b2;
+  void* c2;
 };
 
 __device__ __forceinline__ long crow(const GemmArgs& p, int m) {

@@ -50,6 +50,7 @@ SIGNATURES = {
     "svla_init": [],
     "svla_rmsnorm_bf16": [_p, _i, _p, _p, _i, _i, _i, _f, _p],
     "svla_rmsnorm_rope_table_bf16": [_p, _i, _p, _p, _i, _i, _i, _f, _p, _p, _i, _i, _f, _p],
+    "svla_linear_pair_bf16": [_p, _p, _i, _p, _p, _i, _p, _p, _i, _i, _i, _i, _p],
     "svla_layernorm_bf16": [_p, _i, _p, _p, _p, _i, _i, _i, _f, _p],
     "svla_layernorm_blocked_bf16": [_p, _i, _p, _p, _p, _i, _i, _f, _p],
     "svla_gemm_set_tile": [_i],

@@ -281,6 +281,8 @@ def cross_kv(k_src, v_src, P, out_k=None, out_v=None):
         c = torch.as_strided(out_k, (M, out_k.shape[1] + out_v.shape[1]), (out_k.stride(0), 1))
         ops.linear(a, P["wkvc"], out=c)
         return out_k, out_v
+    if out_k is None and out_v is None:
+        return ops.linear_pair(k_src, P["wkc"], v_src, P["wvc"])
     k = ops.linear(k_src, P["wkc"], out=out_k)
     v = ops.linear(v_src, P["wvc"], out=out_v)
     return k, v

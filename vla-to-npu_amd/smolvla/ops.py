@@ -245,6 +245,22 @@ def linear(a, w, bias=None, bias_f32=None, res=None, act=None, alpha=1.0, out=No
     return out
 
 
+def linear_pair(a0, w0, a1, w1):
+    """``a0 @ w0.T, a1 @ w1.T`` for operands of one shape and stride, in one
+    launch where that pays (``svla_linear_pair_bf16``); else two
+    :func:`linear` calls."""
+    if (a0.shape != a1.shape or w0.shape != w1.shape or _ld(a0) != _ld(a1) or _ld(w0) != _ld(w1)
+            or w0.shape[1] != a0.shape[1]):
+        return linear(a0, w0), linear(a1, w1)
+    M, K = a0.shape
+    N = w0.shape[0]
+    c0 = torch.empty(M, N, dtype=BF16, device=a0.device)
+    c1 = torch.empty_like(c0)
+    _lib.call("svla_linear_pair_bf16", _ptr(a0), _ptr(a1), _ld(a0), _ptr(w0), _ptr(w1), _ld(w0),
+              _ptr(c0), _ptr(c1), N, M, N, K, _stream())
+    return c0, c1
+
+
 LAYOUT_A_BLOCKED, LAYOUT_W_BLOCKED, LAYOUT_C_BLOCKED = 1, 2, 4
 
 
