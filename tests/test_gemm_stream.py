@@ -182,3 +182,23 @@ def test_patch_embed(n, chans, image, patch, embed, pos):
     got = ops.patch_embed(x.cuda(), w.reshape(embed, -1).cuda(), b.cuda(),
                           table.cuda() if pos else None, patch)
     _close(got.view(n, G * G, embed), want, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [5, 9, 17])
+def test_connector_past_256_rows_runs_unsplit(n):
+    """The K split's workspace is one per device: gathers of more than 256 rows
+    leave it alone, so they may overlap on two streams (same bits as with the
+    split turned off)."""
+    from smolvla import _lib, ops
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n, 1024, 768, generator=g).to(BF16).cuda()
+    w = (torch.randn(960, 12288, generator=g) * 0.05).to(BF16).cuda()
+    lib = _lib.load()
+    got = ops.connector(x, w, 4)
+    assert lib.svla_gemm_set_split(1) == 0
+    try:
+        want = ops.connector(x, w, 4)
+    finally:
+        lib.svla_gemm_set_split(-1)
+    assert torch.equal(got, want)

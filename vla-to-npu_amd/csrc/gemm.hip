@@ -2376,8 +2376,13 @@ int run_gemm(GemmArgs& p, int epi, int act, hipStream_t s, WsKind wk = WS_ALLOCA
       stream_takes(p, epi))
     return stream_run(p, epi, act, s);
   if (AMODE != A_DENSE && g_force_tile < 0 && epi == EPI_STORE && gather_takes(p)) {
-    // (a capture that comes before the workspace exists runs unsplit)
-    const SplitWs* w = (long)p.M * p.N * 2 <= (long)kWsFloats && g_force_split != 1 ? split_ws(s) : nullptr;
+    // K is split only where the skinny tiles' choice is a split too (up to
+    // kSkinnyMaxM rows): the workspace is one per device, so calls that split
+    // must not overlap on two streams, and no other gather may come to need it.
+    // (A capture that comes before the workspace exists runs unsplit.)
+    const bool skinny = t.id == S32 || t.id == S64 || t.id == S16;
+    const int tiles = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn);
+    const SplitWs* w = skinny && pick_split(tiles, p.K, t.bm, t.bn) > 1 ? split_ws(s) : nullptr;
     p.ws = w ? w->part : nullptr;
     return gather_run(p, AMODE, s, (long)kWsFloats);
   }

@@ -10,8 +10,8 @@
 // What bounds it (MI355X, measured with copies of the loop that leave out the
 // DMA, the LDS reads or the MFMAs): a CU's LDS-DMA path moves about 57
 // bytes/clock from L2 in 128-byte pieces of line-aligned rows, 27 in 64-byte
-// pieces and 30 when the rows straddle lines (K = 720 rows of 1440 bytes, the
-// reason why layers.py pads the expert's operands to 768 columns).  Per 64-deep
+// pieces and 30 when the rows straddle lines (K = 720, rows of 1440 bytes: the
+// expert's Q, QKV and gate|up operands, about 1 us each).  Per 64-deep
 // K stage a 128x128 tile needs 575 clocks of DMA and 512 of MFMA; 4 waves that
 // each do both halves of a stage in turn (reads, wait, MFMAs) take 1100, since
 // one wave per SIMD cannot overlap its own chain.  So:
@@ -607,13 +607,14 @@ bool gather_takes(const GemmArgs& p) {
          !p.res && !p.norm_w;
 }
 
-// Batched gathers take large tiles, unsplit; a few images' connector has tens
-// of tiles and K = 12288, so its K is split over workgroups as far as the
-// workspace of `ws_floats` floats holds the partial tiles.  MI355X, graph
-// replay, before (64x64 line tile, register-staged 128x128 or split skinny
-// tiles) / now: connector of 1 image 21.6 / 13.8 us, 3 images 40.3 / 19.5, 9
-// images 102 / 32, 32 images 133 / 64, 96 images 250 / 158; patch embedding of
-// 1 image 12.3 / 8.7, 7 images 26.7 / 16.6, 96 images 245 / 174.
+// Unsplit without a workspace; a few images' connector has tens of tiles and
+// K = 12288, so with one its K is split over workgroups as far as `ws_floats`
+// floats hold the partial tiles.  MI355X, graph replay, before (64x64 line
+// tile, register-staged 128x128 or split skinny tiles) / now: connector of 1
+// image 22.0 / 13.9 us, 3 images 40.4 / 21.5, 4 images 42.1 / 23.8 (split), 9
+// images 103 / 60, 32 images 133 / 89 (unsplit; 32 and 64 split, but these
+// never shared the workspace), 96 images 225 / 144; patch embedding of 1 image
+// 12.3 / 8.7, 7 images 26.7 / 16.6, 96 images 245 / 174.
 int gather_run(const GemmArgs& p, int amode, hipStream_t s, long ws_floats) {
   const GatherCfg* best = nullptr;
   int splits = 1;
