@@ -50,3 +50,28 @@ def test_views_and_inputs_kept():
     pv = vit_layer_params(g, VitConfig())
     _same(lambda x: vision_block(x, pv), x_of(1, 196, 768))
     _same(lambda x: vision_block(x, pv), x_of(12, 1024, 768))   # every projection slab-blocked
+
+
+@pytest.mark.parametrize("L", [64, 65, 100])
+def test_rows_on_lines(L):
+    """Weights and norm outputs whose rows start on 128-byte lines give the
+    bits of packed ones (below and from LINE_MIN_ROWS)."""
+    from smolvla import layers
+    from smolvla.vla.action_expert_bf16 import DEFAULT_CFG as cfg
+    g = _Gen(6, device="cuda", norm_init="random")
+    rope = layers.Rope.make(L, cfg.head_dim, cfg.rope_theta, "cuda")
+    x = torch.randn(L, cfg.hidden, device="cuda").to(BF16)
+    p = decoder_layer_params(g, cfg)
+    c = expert_cross_layer_params(g, cfg, 320)
+    ck, cv = (torch.randn(70, cfg.kv_dim, device="cuda").to(BF16) for _ in range(2))
+    got = []
+    for rows in (0, L):
+        P, C = layers.prep_decoder(p, "cuda", rows=rows), layers.prep_cross(c, "cuda", rows=rows)
+        padded = rows >= layers.LINE_MIN_ROWS
+        assert all((w.stride(0) == 768) == padded for w in (P["wqkv"], P["wgu"], C["wq"], C["wgu"]))
+        y = x.clone()
+        kv = layers.decoder_layer(y, P, cfg, 1, L, rope)
+        z = x.clone()
+        layers.cross_layer(z, ck, cv, C, cfg, 1, L, 70, rope)
+        got.append((y, kv, z))
+    assert all(torch.equal(a, b) for a, b in zip(*got))

@@ -75,22 +75,45 @@ def _pack_cols(ws, device):
     return out
 
 
-def prep_decoder(p, device):
-    """SmolLM2 decoder / expert self layer: fused QKV [q|k|v, H], O, gate|up, down."""
+# The mid-size GEMMs read 128-byte pieces of their operands' rows: a piece of a
+# row that starts on a 128-byte line is one line, of others (K = 720: 1440-byte
+# rows) two.  MI355X, graph replay, rows as packed / on lines: batch-32 chunk
+# 38.54 / 38.02 ms; norm outputs alone, expert self layer 32x50 74.3 / 73.2 us.
+# Up to 64 rows packed ones stay: the skinny tiles are faster on them.
+LINE_MIN_ROWS = 65
+
+
+def _line_empty(rows, cols, device):
+    """An uninitialised ``[rows, cols]`` whose rows start on 128-byte lines."""
+    return torch.empty(rows, (cols + 63) // 64 * 64, dtype=BF16, device=device)[:, :cols]
+
+
+def _line_rows(w):
+    """``w`` with every row on a 128-byte line (a copy if it has to be)."""
+    return w if w.shape[1] % 64 == 0 else _line_empty(*w.shape, w.device).copy_(w)
+
+
+def prep_decoder(p, device, rows=0):
+    """SmolLM2 decoder / expert self layer: fused QKV [q|k|v, H], O, gate|up, down.
+    ``rows``: see :func:`prep_cross`."""
+    line = _line_rows if rows >= LINE_MIN_ROWS else lambda w: w
     return dict(
-        wqkv=_pack_cols([p["Wq"], p["Wk"], p["Wv"]], device),
+        wqkv=line(_pack_cols([p["Wq"], p["Wk"], p["Wv"]], device)),
         wo=ops.pack_weight(_dev(p["Wo"], device)),
-        wgu=ops.pack_gate_up(_dev(p["W_gate"], device), _dev(p["W_up"], device)),
+        wgu=line(ops.pack_gate_up(_dev(p["W_gate"], device), _dev(p["W_up"], device))),
         wd=ops.pack_weight(_dev(p["W_down"], device)),
         n1=_dev(p["W_norm_1"], device), n2=_dev(p["W_norm_2"], device),
     )
 
 
-def prep_cross(p, device):
+def prep_cross(p, device, rows=0):
     """Expert cross layer: Q, the cross K/V projections, O, gate|up, down.
     ``wkvc`` packs both cross projections block-diagonally ([K | V] of the
     prefix cache -> [K' | V'] in one GEMM; the zero blocks add exact zeros, so
-    the products equal the two separate GEMMs')."""
+    the products equal the two separate GEMMs').  ``rows`` (the engine's row
+    count, where the fused expert does not read the weights): from
+    ``LINE_MIN_ROWS`` the rows of Q and gate|up start on 128-byte lines."""
+    line = _line_rows if rows >= LINE_MIN_ROWS else lambda w: w
     wk, wv = _dev(p["Wk_cross"], device), _dev(p["Wv_cross"], device)
     kin, kout = wk.shape
     vin, vout = wv.shape
@@ -98,12 +121,12 @@ def prep_cross(p, device):
     wbd[:kin, :kout] = wk
     wbd[kin:, kout:] = wv
     return dict(
-        wq=ops.pack_weight(_dev(p["Wq"], device)),
+        wq=line(ops.pack_weight(_dev(p["Wq"], device))),
         wkc=ops.pack_weight(wk),
         wvc=ops.pack_weight(wv),
         wkvc=ops.pack_weight(wbd.contiguous()),
         wo=ops.pack_weight(_dev(p["Wo"], device)),
-        wgu=ops.pack_gate_up(_dev(p["W_gate"], device), _dev(p["W_up"], device)),
+        wgu=line(ops.pack_gate_up(_dev(p["W_gate"], device), _dev(p["W_up"], device))),
         wd=ops.pack_weight(_dev(p["W_down"], device)),
         n1=_dev(p["W_norm_1"], device), n2=_dev(p["W_norm_2"], device),
     )
@@ -138,11 +161,12 @@ def prep_vit(p, device, rows=None):
 
 VIT_PROJ = {"qkv": "wqkv", "o": "wo", "up": "wup", "down": "wd"}
 
-# The 256x256 GEMM on slab-blocked operands beats the automatic tile choice on
-# row-major operands once a projection has at least this many 256x256 output
-# tiles (MI355X, the SigLIP shapes at 1-10 images of 3 cameras: QKV wins from
-# 216 tiles and loses at 108, O and down win from 144 and lose at 108, the
-# up-projection wins from 144).
+# The 256x256 GEMM on slab-blocked operands against the automatic choice on
+# row-major ones, by 256x256 output tiles (MI355X, SigLIP shapes, graph replay,
+# automatic / blocked us): 108 tiles QKV 17.5 / 22.3, O 19.2 / 26.7, down 46.7 /
+# 67.3; 144 tiles up 27.6 / 26.0, O 27.0 / 27.6, down 72.5 / 69.4; 216 tiles QKV
+# 31.6 / 25.4, O 36.3 / 30.5, down 92.5 / 77.2; past that blocked wins or is
+# within 3% but for one shape (up at 288 tiles, 44.3 / 49.4).
 WIDE_MIN_TILES = 144
 
 
@@ -153,11 +177,9 @@ def vit_blocked_plan(hidden: int, inter: int, rows: int) -> dict:
     up-projection then read a slab-blocked LayerNorm output; the
     down-projection reads the up-projection's output slab-blocked, so it goes
     blocked only together with the up-projection; O reads the attention
-    output row-major.  A projection the plan moves gives the same bits on
-    either path (measured at 3 and 12 images: the automatic tiles it replaces
-    accumulate K in the same order); only the 96x96 tile the batch-1
-    down-projection keeps sums in another order, which the plan never
-    replaces."""
+    output row-major.  A projection the plan moves may differ from
+    the automatic path by a rounding: the K-split tiles add the two halves of
+    every 64-deep K stage separately."""
     shapes = {"qkv": (3 * hidden, hidden), "o": (hidden, hidden),
               "up": (inter, hidden), "down": (hidden, inter)}
     plan = {name: (rows % 256 == 0 and n % 256 == 0 and k % 128 == 0 and k >= 256 and
@@ -193,10 +215,11 @@ class Buffers:
         self.device = device
         self._b = {}
 
-    def get(self, name, rows, cols, dtype=BF16):
+    def get(self, name, rows, cols, dtype=BF16, line=False):
         t = self._b.get(name)
         if t is None or t.shape[0] < rows or t.shape[1] != cols or t.dtype != dtype:
-            t = torch.empty(rows, cols, dtype=dtype, device=self.device)
+            t = (_line_empty(rows, cols, self.device) if line
+                 else torch.empty(rows, cols, dtype=dtype, device=self.device))
             self._b[name] = t
         return t[:rows]
 
@@ -214,11 +237,11 @@ def _normed(x, w, eps, M, bufs, name, rope=None):
     theta = rope.theta if rope is not None else None
     if theta is not None:
         rope.theta = None
-        out = bufs.get(name, M, x.shape[1])
+        out = bufs.get(name, M, x.shape[1], line=M >= LINE_MIN_ROWS)
         return ops.rmsnorm_rope_table(x, w, eps, rope.cos, rope.sin, theta, out=out), None
     if M <= FUSED_NORM_MAX_ROWS:
         return x, (w, eps)
-    return ops.rmsnorm(x, w, eps, out=bufs.get(name, M, x.shape[1])), None
+    return ops.rmsnorm(x, w, eps, out=bufs.get(name, M, x.shape[1], line=M >= LINE_MIN_ROWS)), None
 
 
 def decoder_layer(x, P, cfg: DecoderConfig, B, L, rope: Rope, mask="causal", prefix_len=0,

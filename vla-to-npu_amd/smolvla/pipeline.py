@@ -73,7 +73,8 @@ class SmolVLAEngine:
         self.embed_table = pd(P["embed"])
         self.state_w = ops.pack_weight(pd(P["state"]["W"]))
         self.prefix = [layers.prep_decoder(lp, dev) for lp in P["prefix"]]
-        self.expert = [layers.prep_cross(lp, dev) if cfg.is_cross(i) else layers.prep_decoder(lp, dev)
+        rows = 0 if self.fused_expert else self.B * cfg.chunk
+        self.expert = [(layers.prep_cross if cfg.is_cross(i) else layers.prep_decoder)(lp, dev, rows=rows)
                        for i, lp in enumerate(P["expert"])]
         io = P["expert_io"]
         H = e.hidden
