@@ -12,9 +12,9 @@
 // GEMM or attention of the step sequence) that every workgroup walks.
 //
 // Design (CDNA4; the figures are MI355X measurements of this build):
-//  * One workgroup of 8 waves per CU.  A phase is split into UNITS (a
-//    64-row x 16-column output tile of a GEMM, one (sample, head) of an
-//    attention); unit u of a phase runs on team rank u % team_size.
+//  * One workgroup of 8 waves per CU.  A phase is split into UNITS (an
+//    output tile of a GEMM: the whole rows x 16 columns, or 32 x 32 for paired
+//    projections; one (sample, head) of an attention); unit u of a phase runs on team rank u % team_size.
 //  * Phases hand over through device-scope arrival counters: a workgroup
 //    that finished its units of phase p waits for its stores to be
 //    acknowledged (vmcnt = 0), then adds its unit count to one of 16

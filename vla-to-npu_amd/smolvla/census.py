@@ -181,7 +181,7 @@ class Group:
 
 # entry points that set state rather than launch work: not timed
 _SKIP = {"svla_init", "svla_version", "svla_gemm_set_tile", "svla_gemm_set_split",
-         "svla_gemm_tile_choice", "svla_expert_workspace_size", "svla_expert_prepare",
+         "svla_gemm_tile_choice", "svla_gemm_stream_choice", "svla_expert_workspace_size", "svla_expert_prepare",
          "svla_expert_status", "svla_time_embedding_bf16", "svla_rope_table"}
 
 
@@ -290,6 +290,7 @@ _FAMILIES = {
     "svla_layernorm_blocked_bf16": [("layernorm_kernel",)],
 }
 _GEMM = ("gemm_", "skinny_kernel")
+_GEMM_TAIL = "stream_reduce_kernel"   # sums a gather's K parts, after its GEMM
 
 
 def dispatch_families(name):
@@ -327,15 +328,24 @@ def align_last_chunk(calls, dispatches):
     returns [(call index, dispatch row)]; raises if a kernel family does not
     match its call."""
     fam = [(i, f) for i, c in enumerate(calls) for f in dispatch_families(c[0])]
-    if len(dispatches) < len(fam):
-        raise ValueError(f"{len(dispatches)} dispatches for {len(fam)} expected")
-    tail = dispatches[len(dispatches) - len(fam):]
+    # the second dispatch of a K-split gather belongs to the gather's call
+    main, extra = [], {}
+    for r in dispatches:
+        if main and short_kernel_name(r["Kernel_Name"]).startswith(_GEMM_TAIL):
+            extra[len(main) - 1] = r
+        else:
+            main.append(r)
+    if len(main) < len(fam):
+        raise ValueError(f"{len(main)} dispatches for {len(fam)} expected")
+    first = len(main) - len(fam)
     out = []
-    for (i, f), r in zip(fam, tail):
-        k = short_kernel_name(r["Kernel_Name"])
+    for n, (i, f) in enumerate(fam, first):
+        k = short_kernel_name(main[n]["Kernel_Name"])
         if not k.startswith(f):
             raise ValueError(f"call {i} ({calls[i][0]}) expects {f}, profiler shows {k}")
-        out.append((i, r))
+        out.append((i, main[n]))
+        if n in extra:
+            out.append((i, extra[n]))
     return out
 
 
