@@ -1,0 +1,44 @@
+"""The packed weights that the layer functions keep between calls: CPU checks
+of when a call packs (preparation and launches replaced by stand-ins)."""
+
+import pytest
+import torch
+
+from smolvla import layers
+from smolvla.config import VitConfig
+from smolvla.vla import vision_block_bf16
+
+
+@pytest.fixture
+def packs(monkeypatch):
+    """vision_block on CPU tensors, its launches left out; returns the calls
+    of prep_vit."""
+    calls = []
+
+    def prep(p, device, rows=None):
+        calls.append(rows)
+        return dict(p)
+
+    monkeypatch.setattr(vision_block_bf16, "to_device", lambda x: (x, lambda t: t))
+    monkeypatch.setattr(layers, "prep_vit", prep)
+    monkeypatch.setattr(layers, "vit_layer", lambda *a, **k: None)
+    return calls
+
+
+def test_vision_block_packs_once_for_every_size(packs):
+    """No call size may find its weights unpacked after a call of another: it
+    may come inside a graph capture, where packing would only be recorded."""
+    params = {"Wq": torch.zeros(8, 768), "W_up": torch.zeros(8, 3072)}
+    for rows in (196, 4 * 1024, 1024, 12 * 1024, 96 * 1024 + 64):
+        x = torch.empty(1, rows, 768, dtype=torch.bfloat16)
+        vision_block_bf16.vision_block(x, params, VitConfig())
+    assert len(packs) == 1
+
+
+@pytest.mark.parametrize("hidden,inter", [(768, 3072), (768, 384), (1152, 4304), (128, 256)])
+def test_blockable_is_the_plan_at_large_calls(hidden, inter):
+    fits = layers.vit_blockable(hidden, inter)
+    assert fits == layers.vit_blocked_plan(hidden, inter, 256 * layers.WIDE_MIN_TILES)
+    for rows in (256, 3072, 4096, 12288, 12300):
+        plan = layers.vit_blocked_plan(hidden, inter, rows)
+        assert all(fits[k] or not plan[k] for k in plan)

@@ -1,0 +1,38 @@
+"""Packed weights kept between layer calls, where a call comes inside a graph
+capture or on another stream than the one that packed."""
+
+import pytest
+import torch
+
+from smolvla.params import _Gen, vit_layer_params
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def _capture(fn):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fn()
+    return graph, out
+
+
+def test_vision_block_capture_after_a_warm_up_of_another_size():
+    """One small eager call, then a capture of a size on the slab-blocked
+    GEMM: an eager call before the first replay, and every replay, give the
+    bits of a call whose weights were packed in the open."""
+    from smolvla.config import VitConfig
+    from smolvla.vla.vision_block_bf16 import vision_block
+    g = _Gen(9, device="cuda", norm_init="random")
+    params = vit_layer_params(g, VitConfig())
+    x = torch.randn(4, 1024, 768, device="cuda").to(BF16)
+    want = vision_block(x, dict(params))
+    vision_block(x[:1, :196], params)
+    graph, out = _capture(lambda: vision_block(x, params))
+    assert torch.equal(vision_block(x, params), want)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(vision_block(x, params), want)

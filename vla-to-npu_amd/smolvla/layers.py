@@ -135,7 +135,8 @@ def prep_cross(p, device, rows=0):
 def prep_vit(p, device, rows=None):
     """Packed ViT block weights.  ``rows`` (the engine's row count, images x
     tokens): also slab-blocked copies of the weights that
-    :func:`vit_blocked_plan` puts on the 256x256 GEMM at that row count."""
+    :func:`vit_blocked_plan` puts on the 256x256 GEMM at that row count, or
+    with ``ANY_ROWS`` at some row count."""
     H = p["Wq"].shape[0]
     bqkv = None
     if p.get("bq") is not None:
@@ -152,12 +153,15 @@ def prep_vit(p, device, rows=None):
         g2=_dev(p["W_norm_2"], device), b2=opt("b_norm_2"),
     )
     if rows:
-        plan = vit_blocked_plan(H, P["wup"].shape[0], rows)
+        inter = P["wup"].shape[0]
+        plan = vit_blockable(H, inter) if rows is ANY_ROWS else vit_blocked_plan(H, inter, rows)
         for k, w in VIT_PROJ.items():
             if plan[k]:
                 P[w + "_blk"] = ops.slab_block(P[w])
     return P
 
+
+ANY_ROWS = "any"    # prep_vit: weights for calls of every row count
 
 VIT_PROJ = {"qkv": "wqkv", "o": "wo", "up": "wup", "down": "wd"}
 
@@ -180,13 +184,27 @@ def vit_blocked_plan(hidden: int, inter: int, rows: int) -> dict:
     output row-major.  A projection the plan moves may differ from
     the automatic path by a rounding: the K-split tiles add the two halves of
     every 64-deep K stage separately."""
-    shapes = {"qkv": (3 * hidden, hidden), "o": (hidden, hidden),
-              "up": (inter, hidden), "down": (hidden, inter)}
-    plan = {name: (rows % 256 == 0 and n % 256 == 0 and k % 128 == 0 and k >= 256 and
+    fits = vit_blockable(hidden, inter)
+    plan = {name: (fits[name] and rows % 256 == 0 and
                    (rows // 256) * (n // 256) >= WIDE_MIN_TILES)
-            for name, (n, k) in shapes.items()}
+            for name, (n, _) in _vit_shapes(hidden, inter).items()}
     plan["down"] = plan["down"] and plan["up"]
     return plan
+
+
+def _vit_shapes(hidden, inter):
+    """(output columns, depth) of the ViT projections."""
+    return {"qkv": (3 * hidden, hidden), "o": (hidden, hidden),
+            "up": (inter, hidden), "down": (hidden, inter)}
+
+
+def vit_blockable(hidden: int, inter: int) -> dict:
+    """The projections that :func:`vit_blocked_plan` can move at some row
+    count: those whose columns and depth the 256x256 GEMM takes."""
+    fits = {name: n % 256 == 0 and k % 128 == 0 and k >= 256
+            for name, (n, k) in _vit_shapes(hidden, inter).items()}
+    fits["down"] = fits["down"] and fits["up"]
+    return fits
 
 
 @dataclass

@@ -24,11 +24,14 @@ FFN_HID = 3072
 DEFAULT_CFG = VitConfig()
 
 
-def _prep_blocked(p, device):
-    """Weights for calls whose rows put projections on the slab-blocked
-    256x256 GEMM: blocked copies of every projection that a large enough call
-    moves there (each call's own plan picks among them)."""
-    return layers.prep_vit(p, device, rows=1 << 20)
+def _prep_any_rows(p, device):
+    """One set of packed weights for calls of every size: beside the row-major
+    ones blocked copies of every projection that a large enough call moves to
+    the slab-blocked 256x256 GEMM (each call's own plan picks among them).  The
+    first call, whatever its size, then packs for all others: one of another
+    size finds nothing left to pack, also where it must not (under capture, or
+    beside calls on other streams)."""
+    return layers.prep_vit(p, device, rows=layers.ANY_ROWS)
 
 
 def vision_block(x_np, params, cfg: VitConfig = DEFAULT_CFG):
@@ -36,8 +39,7 @@ def vision_block(x_np, params, cfg: VitConfig = DEFAULT_CFG):
     x3, squeeze = as_batched(x)
     B, T, H = x3.shape
     x2 = as_rows(x3)
-    plan = layers.vit_blocked_plan(H, params["W_up"].shape[1], B * T)
-    P = prepared(params, _prep_blocked if any(plan.values()) else layers.prep_vit)
+    P = prepared(params, _prep_any_rows)
     out = torch.empty_like(x2)
     layers.vit_layer(x2, P, cfg, B, T, out=out)
     return back(out.view(T, H) if squeeze else out.view(B, T, H))
