@@ -6,7 +6,7 @@ import torch
 
 from smolvla import layers
 from smolvla.config import VitConfig
-from smolvla.vla import vision_block_bf16
+from smolvla.vla import _common, vision_block_bf16
 
 
 @pytest.fixture
@@ -42,3 +42,19 @@ def test_blockable_is_the_plan_at_large_calls(hidden, inter):
     for rows in (256, 3072, 4096, 12288, 12300):
         plan = layers.vit_blocked_plan(hidden, inter, rows)
         assert all(fits[k] or not plan[k] for k in plan)
+
+
+def test_what_a_capture_packs_is_not_kept(monkeypatch):
+    """Packing inside a graph capture is recorded, not run: a later call may
+    not take its tensors for packed weights, nor lose an entry to them."""
+    calls = []
+    pack = lambda p, device: calls.append(p) or len(calls)  # noqa: E731
+    params, kept = {"W": torch.ones(2)}, {"W": torch.zeros(2)}
+    assert _common.prepared(kept, pack) == 1
+    monkeypatch.setattr(_common, "_capturing", lambda: True, raising=False)
+    assert _common.prepared(params, pack) == 2
+    assert _common.prepared(params, pack) == 3              # one graph's, not another's
+    assert _common.prepared(kept, pack) == 1                # packed before: used as it is
+    monkeypatch.setattr(_common, "_capturing", lambda: False, raising=False)
+    assert _common.prepared(params, pack) == 4              # an eager call packs its own
+    assert _common.prepared(params, pack) == 4 and len(calls) == 4

@@ -4,7 +4,7 @@ capture or on another stream than the one that packed."""
 import pytest
 import torch
 
-from smolvla.params import _Gen, vit_layer_params
+from smolvla.params import _Gen, decoder_layer_params, vit_layer_params
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -36,3 +36,27 @@ def test_vision_block_capture_after_a_warm_up_of_another_size():
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         assert torch.equal(vision_block(x, params), want)
+
+
+def test_capture_with_no_call_before():
+    """Weights never packed before the capture: the graph packs them itself on
+    every replay, and an eager call, before and after, packs its own."""
+    from smolvla.config import DecoderConfig
+    from smolvla.vla.text_encoder_bf16 import text_encoder_forward
+    g = _Gen(10, device="cuda", norm_init="random")
+    params = decoder_layer_params(g, DecoderConfig())
+    x = torch.randn(2, 37, 960, device="cuda").to(BF16)
+    want = text_encoder_forward(x, dict(params))
+    graph, out = _capture(lambda: text_encoder_forward(x, params))
+
+    def same(got):
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+    same(text_encoder_forward(x, params))
+    for _ in range(3):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        same(out)
+        same(text_encoder_forward(x, params))

@@ -59,7 +59,9 @@ def as_rows(x3):
 # caller's dict: an entry is reused only while the dict holds the very same
 # weight objects with unchanged contents (torch tensors: the version counter
 # every in-place update bumps; numpy arrays: a content hash), so an updated
-# weight is re-packed, never served stale.
+# weight is re-packed, never served stale.  What is packed while a graph is
+# being captured is not kept: it is only recorded, into memory of that graph,
+# and is written when the graph is replayed.
 _PREPARED = collections.OrderedDict()
 _PREPARED_MAX = 64
 
@@ -79,9 +81,14 @@ def _state(params):
     return vals, tuple(marks)
 
 
+def _capturing():
+    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+
+
 def prepared(params, prep_fn):
     """Pack reference-layout weights (torch tensors or the reference's numpy
-    arrays, ``[in, out]``) once per params dict and weight state."""
+    arrays, ``[in, out]``) once per params dict and weight state (inside a
+    graph capture: once per call, by the graph itself)."""
     key = (id(params), prep_fn)
     vals, marks = _state(params)
     hit = _PREPARED.get(key)
@@ -90,6 +97,8 @@ def prepared(params, prep_fn):
         _PREPARED.move_to_end(key)
         return hit[2]
     out = prep_fn(params, torch.device("cuda"))
+    if _capturing():
+        return out
     _PREPARED[key] = (vals, marks, out)     # holds the weight objects: ids stay unique
     _PREPARED.move_to_end(key)
     while len(_PREPARED) > _PREPARED_MAX:
