@@ -58,3 +58,48 @@ def test_what_a_capture_packs_is_not_kept(monkeypatch):
     monkeypatch.setattr(_common, "_capturing", lambda: False, raising=False)
     assert _common.prepared(params, pack) == 4              # an eager call packs its own
     assert _common.prepared(params, pack) == 4 and len(calls) == 4
+
+
+class _Stream:
+    def __init__(self):
+        self.waited = []
+
+    def wait_event(self, event):
+        self.waited.append(event)
+
+
+class _Event:
+    def record(self):
+        self.stream = torch.cuda.current_stream()
+
+
+def test_another_stream_waits_for_the_packing(monkeypatch):
+    """The first hit on another stream than the one that packed waits for the
+    packing; a hit inside a capture does not."""
+    here, there, third = _Stream(), _Stream(), _Stream()
+    cur = [here]
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: cur[0])
+    monkeypatch.setattr(_common, "_raw_stream", lambda: id(cur[0]), raising=False)
+    monkeypatch.setattr(torch.cuda, "Event", _Event)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    recorded = []
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: recorded.append((t, s)))
+    params, w = {"W": torch.ones(2)}, torch.ones(3)
+    pack = lambda p, device: dict(w=w, b=None)  # noqa: E731
+    _common.prepared(params, pack)
+    _common.prepared(params, pack)
+    assert not here.waited and not recorded
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    cur[0] = there
+    _common.prepared(params, pack)
+    assert not there.waited
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    for _ in range(2):
+        _common.prepared(params, pack)
+    assert [e.stream for e in there.waited] == [here]
+    assert len(recorded) == 1 and recorded[0][0] is w and recorded[0][1] is there
+    cur[0] = third
+    _common.prepared(params, pack)
+    assert [e.stream for e in third.waited] == [here] and len(recorded) == 2
+    assert not here.waited

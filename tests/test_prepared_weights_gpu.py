@@ -60,3 +60,24 @@ def test_capture_with_no_call_before():
         torch.cuda.synchronize()
         same(out)
         same(text_encoder_forward(x, params))
+
+
+def test_a_call_on_another_stream_waits_for_the_packing():
+    """The first call packs behind other work of its stream; a call on a second
+    stream, made at once, gives the same bits."""
+    from smolvla.vla.action_expert_bf16 import DEFAULT_CFG, action_expert_self_forward
+    g = _Gen(11, device="cuda", norm_init="random")
+    params = decoder_layer_params(g, DEFAULT_CFG)
+    x = torch.randn(2, 50, 720, device="cuda").to(BF16)
+    want = action_expert_self_forward(x, dict(params))
+    busy = torch.randn(8192, 8192, device="cuda")
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        for _ in range(4):
+            busy = busy @ busy * 1e-4
+        a = action_expert_self_forward(x, params)
+    with torch.cuda.stream(second):
+        b = action_expert_self_forward(x, params)
+    torch.cuda.synchronize()
+    assert torch.equal(a, want) and torch.equal(b, want)

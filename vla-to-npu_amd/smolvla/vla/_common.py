@@ -85,6 +85,43 @@ def _capturing():
     return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
 
 
+def _raw_stream():
+    """The current stream's handle (0.5 us; a Stream object takes 2.6)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+class _Packed:
+    """A kept set of packed weights.  It is written on the stream that was
+    current then; the first call on another stream waits for that, and tells
+    the allocator, so that memory of a dropped set is not handed out under it."""
+
+    def __init__(self, vals, marks, out):
+        self.vals, self.marks, self.out = vals, marks, out   # vals: ids stay unique
+        self.streams, self.event = (), None
+        if torch.cuda.is_available():
+            self.streams = (_raw_stream(),)
+            self.event = torch.cuda.Event()
+            self.event.record()
+
+    def holds(self, vals, marks):
+        return (self.marks == marks and len(self.vals) == len(vals)
+                and all(a is b for a, b in zip(self.vals, vals)))
+
+    def use(self):
+        if not self.streams:
+            return self.out             # no GPU
+        raw = _raw_stream()
+        if raw in self.streams or _capturing():
+            return self.out             # (a capture may not wait for work outside it)
+        stream = torch.cuda.current_stream()
+        stream.wait_event(self.event)
+        for t in self.out.values() if isinstance(self.out, dict) else (self.out,):
+            if torch.is_tensor(t):
+                t.record_stream(stream)
+        self.streams += (raw,)
+        return self.out
+
+
 def prepared(params, prep_fn):
     """Pack reference-layout weights (torch tensors or the reference's numpy
     arrays, ``[in, out]``) once per params dict and weight state (inside a
@@ -92,14 +129,13 @@ def prepared(params, prep_fn):
     key = (id(params), prep_fn)
     vals, marks = _state(params)
     hit = _PREPARED.get(key)
-    if hit is not None and hit[1] == marks and len(hit[0]) == len(vals) and all(
-            a is b for a, b in zip(hit[0], vals)):
+    if hit is not None and hit.holds(vals, marks):
         _PREPARED.move_to_end(key)
-        return hit[2]
+        return hit.use()
     out = prep_fn(params, torch.device("cuda"))
     if _capturing():
         return out
-    _PREPARED[key] = (vals, marks, out)     # holds the weight objects: ids stay unique
+    _PREPARED[key] = _Packed(vals, marks, out)
     _PREPARED.move_to_end(key)
     while len(_PREPARED) > _PREPARED_MAX:
         _PREPARED.popitem(last=False)
