@@ -31,3 +31,15 @@ def test_down_goes_blocked_only_with_up():
     plan = layers.vit_blocked_plan(768, 384, 12288)
     assert not plan["up"] and not plan["down"]
     assert plan["qkv"] and plan["o"]
+
+
+@pytest.mark.parametrize("rows, want", [
+    ((1 << 31) // 3072 // 256 * 256, ALL),                     # the last rows under 2^31 elements
+    ((1 << 31) // 3072 // 256 * 256 + 256, ALL - {"down"}),
+    (684 * 1024, ALL - {"down"}),                              # 228 samples of 3 cameras
+    ((1 << 31) // 768 // 256 * 256 + 256, set()),
+])
+def test_operands_past_the_kernels_limit_stay_row_major(rows, want):
+    """svla_linear_wide_bf16 refuses operands of more than 2^31 elements."""
+    plan = layers.vit_blocked_plan(768, 3072, rows)
+    assert {k for k, v in plan.items() if v} == want

@@ -172,6 +172,9 @@ VIT_PROJ = {"qkv": "wqkv", "o": "wo", "up": "wup", "down": "wd"}
 # 31.6 / 25.4, O 36.3 / 30.5, down 92.5 / 77.2; past that blocked wins or is
 # within 3% but for one shape (up at 288 tiles, 44.3 / 49.4).
 WIDE_MIN_TILES = 144
+# the most elements of an operand that svla_linear_wide_bf16 takes; larger ones
+# stay on the automatic choice, which has no such limit
+WIDE_MAX_ELEMS = 1 << 31
 
 
 def vit_blocked_plan(hidden: int, inter: int, rows: int) -> dict:
@@ -185,9 +188,9 @@ def vit_blocked_plan(hidden: int, inter: int, rows: int) -> dict:
     the automatic path by a rounding: the K-split tiles add the two halves of
     every 64-deep K stage separately."""
     fits = vit_blockable(hidden, inter)
-    plan = {name: (fits[name] and rows % 256 == 0 and
+    plan = {name: (fits[name] and rows % 256 == 0 and rows * k <= WIDE_MAX_ELEMS and
                    (rows // 256) * (n // 256) >= WIDE_MIN_TILES)
-            for name, (n, _) in _vit_shapes(hidden, inter).items()}
+            for name, (n, k) in _vit_shapes(hidden, inter).items()}
     plan["down"] = plan["down"] and plan["up"]
     return plan
 
@@ -201,7 +204,8 @@ def _vit_shapes(hidden, inter):
 def vit_blockable(hidden: int, inter: int) -> dict:
     """The projections that :func:`vit_blocked_plan` can move at some row
     count: those whose columns and depth the 256x256 GEMM takes."""
-    fits = {name: n % 256 == 0 and k % 128 == 0 and k >= 256
+    fits = {name: (n % 256 == 0 and k % 128 == 0 and k >= 256 and
+                   n * k <= WIDE_MAX_ELEMS)
             for name, (n, k) in _vit_shapes(hidden, inter).items()}
     fits["down"] = fits["down"] and fits["up"]
     return fits
