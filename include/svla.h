@@ -233,9 +233,18 @@ int svla_gemm_tile_choice(int m, int n, int k, int act);
  * names.  These kernels are not among the forceable configurations. */
 int svla_gemm_stream_choice(int m, int n, int k, int paired);
 
+/* Query: K splits * 1000000 + block tile (rows * 1000 + columns) with which a
+ * patch embedding or connector of m rows, n columns (multiples of 8) and depth k
+ * runs while the split-K workspace exists, or 0 where a tile is forced.  m >= 64,
+ * k >= 64 (smaller ones run on the configurations of svla_gemm_set_tile). */
+int svla_gemm_gather_choice(int m, int n, int k);
+
 /* Tuning hook: force the number of cross-workgroup K splits of skinny
  * (M <= 256) GEMMs, 1..64 (1 = never split), or -1 for the automatic choice
- * (default).  Process-wide; not thread-safe. */
+ * (default).  Counts over 1 hold for the problems whose automatic choice is a
+ * skinny tile, which then keep it, and for the patch embeddings and connectors
+ * of up to 256 rows; a split has at least 32 of K, a gather's 64.
+ * Process-wide; not thread-safe. */
 int svla_gemm_set_split(int splits);
 
 /* Fused (RMSNorm +) QKV projection with rotate-half RoPE in the epilogue.

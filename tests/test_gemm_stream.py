@@ -202,3 +202,81 @@ def test_connector_past_256_rows_runs_unsplit(n):
     finally:
         lib.svla_gemm_set_split(-1)
     assert torch.equal(got, want)
+
+
+@pytest.fixture
+def force_split():
+    from smolvla import _lib
+    lib = _lib.load()
+
+    def force(n):
+        assert lib.svla_gemm_set_split(n) == 0
+    yield force
+    lib.svla_gemm_set_split(-1)
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 960, 12288), (192, 960, 12288), (256, 72, 2048)])
+def test_gathers_obey_a_forced_split(force_split, m, n, k):
+    from smolvla import _lib
+    choice = _lib.load().svla_gemm_gather_choice
+    assert choice(m, n, k) // 1000000 > 1                 # split by themselves
+    for z in (1, 2, 3, 5, 12, 13, 22):
+        force_split(z)
+        assert choice(m, n, k) // 1000000 == z
+
+
+def test_forced_gather_splits_end_at_k_and_at_the_workspace(force_split):
+    from smolvla import _lib
+    choice = _lib.load().svla_gemm_gather_choice
+    force_split(64)
+    assert choice(64, 72, 200) // 1000000 == 4            # a 64-deep stage each
+    # 2^22 floats of partial tiles: 22 times 192 x 960
+    assert choice(192, 960, 12288) // 1000000 == 22
+    assert choice(320, 960, 12288) // 1000000 == 1        # more rows never split
+
+
+def test_dense_skinny_problems_obey_a_forced_split(force_split):
+    """A count over 1 keeps them on the skinny tile, which splits; 1 does not
+    need it."""
+    from smolvla import _lib
+    choice = _lib.load().svla_gemm_stream_choice
+    auto = choice(100, 1600, 960, 1)
+    assert auto > 0
+    for z, want in ((4, 0), (1, auto), (-1, auto)):
+        force_split(z)
+        assert choice(100, 1600, 960, 1) == want
+
+
+@pytest.mark.gpu
+def test_connector_at_forced_splits(force_split):
+    """Every count gives the product, and the counts' sums are their own."""
+    from smolvla import ops
+    ops.init()
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(3, 1024, 768, generator=g).to(BF16)
+    w = (torch.randn(12288, 960, generator=g) * 0.05).to(BF16)
+    t = x.view(3, 8, 4, 8, 4, 768).permute(0, 1, 3, 2, 4, 5).reshape(192, 12288)
+    want = (t.float() @ w.float()).to(BF16)
+    X, W = x.cuda(), ops.pack_weight(w.cuda())
+    got = []
+    for z in (-1, 1, 2, 3, 5, 13, 22):
+        force_split(z)
+        got.append(ops.connector(X, W, 4))
+        _close(got[-1], want)
+    assert all(not torch.equal(a, b) for a, b in zip(got[1:], got[2:]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(100, 1600, 960), (65, 960, 720), (128, 1600, 2048)])
+def test_paired_at_forced_splits(force_split, m, n, k):
+    from smolvla import ops
+    ops.init()
+    g = torch.Generator().manual_seed(m)
+    a = torch.randn(m, k, generator=g).to(BF16)
+    wg, wu = ((torch.randn(k, n // 2, generator=g) * 0.05).to(BF16) for _ in range(2))
+    W = ops.pack_gate_up(wg.cuda(), wu.cuda())
+    gate, up = ((a.float() @ w.float()).to(BF16).float() for w in (wg, wu))
+    s = torch.nn.functional.silu(gate).to(BF16).float()
+    for z in (-1, 1, 2, 4):
+        force_split(z)
+        _close(ops.linear_silu_mul(a.cuda(), W), (s * up).to(BF16), gate * up, up * s)

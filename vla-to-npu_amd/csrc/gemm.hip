@@ -2327,6 +2327,29 @@ bool small_range(int M, int N, int K, int epi) {
   return M > 128 && tiles(32, 64) <= kNumCU;
 }
 
+bool skinny_tile(TileId t) { return t == S32 || t == S64 || t == S16; }
+
+// The K-split line-DMA kernels take the mid-size dense problems: everything but
+// the small tiles' and the 256x256 kernel's own ranges, and skinny problems
+// whose K splits are forced (svla_gemm_set_split).
+bool stream_range(int M, int N, int K, int epi, TileId t) {
+  return g_force_tile < 0 && t != W256 && !(g_force_split > 1 && skinny_tile(t)) &&
+         !small_range(M, N, K, epi);
+}
+
+// Whether a gather may split K: only where the skinny tiles' choice is a split
+// too (up to kSkinnyMaxM rows).  The workspace is one per device, so calls that
+// split must not overlap on two streams, and no other gather may come to need
+// it.  `force`: the count that svla_gemm_set_split names, as far as those tiles
+// take it.
+bool gather_split(int M, int N, int K, const TileCfg& t, int& force) {
+  if (!skinny_tile(t.id)) return false;
+  const int tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+  const int S = pick_split(tiles, K, t.bm, t.bn);
+  force = g_force_split > 1 ? S : 0;
+  return S > 1;
+}
+
 template <int AMODE, bool NORM>
 int dispatch(const GemmArgs& p, int epi, int act, TileId t, dim3 grid, hipStream_t s) {
   int rc;
@@ -2370,21 +2393,14 @@ int run_gemm(GemmArgs& p, int epi, int act, hipStream_t s, WsKind wk = WS_ALLOCA
   const bool wide_rows_ok = !p.out_f32 && p.N % 8 == 0 && p.ldc % 8 == 0 &&
                             (!p.res || (p.ldr % 8 == 0 && svla_aligned16(p.res)));
   const TileCfg t = pick_tile(p.M, p.N, p.K, epi, plain, wide_rows_ok, AMODE == A_DENSE);
-  // the K-split line-DMA kernels take the mid-size dense problems (everything
-  // but the small tiles' and the 256x256 kernel's own ranges)
-  if (AMODE == A_DENSE && g_force_tile < 0 && t.id != W256 && !small_range(p.M, p.N, p.K, epi) &&
-      stream_takes(p, epi))
+  if (AMODE == A_DENSE && stream_range(p.M, p.N, p.K, epi, t.id) && stream_takes(p, epi))
     return stream_run(p, epi, act, s);
   if (AMODE != A_DENSE && g_force_tile < 0 && epi == EPI_STORE && gather_takes(p)) {
-    // K is split only where the skinny tiles' choice is a split too (up to
-    // kSkinnyMaxM rows): the workspace is one per device, so calls that split
-    // must not overlap on two streams, and no other gather may come to need it.
-    // (A capture that comes before the workspace exists runs unsplit.)
-    const bool skinny = t.id == S32 || t.id == S64 || t.id == S16;
-    const int tiles = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn);
-    const SplitWs* w = skinny && pick_split(tiles, p.K, t.bm, t.bn) > 1 ? split_ws(s) : nullptr;
+    // (a capture that comes before the workspace exists runs unsplit)
+    int force = 0;
+    const SplitWs* w = gather_split(p.M, p.N, p.K, t, force) ? split_ws(s) : nullptr;
     p.ws = w ? w->part : nullptr;
-    return gather_run(p, AMODE, s, (long)kWsFloats);
+    return gather_run(p, AMODE, gather_plan(p.M, p.N, p.K, w ? (long)kWsFloats : 0, force), s);
   }
   if (p.norm_w && p.K > 2048) return SVLA_EINVAL;  // the gain vector is staged in LDS (<= 2048)
   // a pipelined kernel needs one full K stage, the wide one whole 4-step
@@ -2404,7 +2420,7 @@ int run_gemm(GemmArgs& p, int epi, int act, hipStream_t s, WsKind wk = WS_ALLOCA
     grid = dim3(min(gm * gn, kNumCU), 1, 1);
     p.w_cn = wide_cols_per_xcd(gm, gn, p.K, (int)grid.x);
   }
-  if (t.id == S32 || t.id == S64 || t.id == S16) {
+  if (skinny_tile(t.id)) {
     const int S = pick_split(gm * gn, p.K, t.bm, t.bn);
     const SplitWs* w = nullptr;
     if (S > 1 && wk == WS_SCRATCH) {
@@ -2470,10 +2486,17 @@ int svla_gemm_tile_choice(int m, int n, int k, int act) {
 int svla_gemm_stream_choice(int m, int n, int k, int paired) {
   if (m <= 0 || n <= 0 || n % (paired ? 64 : 8) || k < 8 || k % 8) return SVLA_EINVAL;
   const int epi = paired ? EPI_ROPE : EPI_STORE;
-  if (g_force_tile >= 0 || pick_tile(m, n, k, epi, !paired, true, true).id == W256 ||
-      small_range(m, n, k, epi))
-    return 0;
+  if (!stream_range(m, n, k, epi, pick_tile(m, n, k, epi, !paired, true, true).id)) return 0;
   return stream_tile(m, n, k, epi);
+}
+
+int svla_gemm_gather_choice(int m, int n, int k) {
+  if (m < 64 || n <= 0 || n % 8 || k < LBK || k % 8) return SVLA_EINVAL;
+  if (g_force_tile >= 0) return 0;
+  int force = 0;
+  const bool split = gather_split(m, n, k, pick_tile(m, n, k, EPI_STORE, false, true, false), force);
+  const GatherPlan g = gather_plan(m, n, k, split ? (long)kWsFloats : 0, force);
+  return g.splits * 1000000 + gather_tile(g);
 }
 
 int svla_gemm_set_split(int splits) {

@@ -128,10 +128,18 @@ __attribute__((visibility("hidden"))) int stream_tile(int M, int N, int K, int e
 __attribute__((visibility("hidden"))) int stream_run(const GemmArgs& p, int epi, int act,
                                                      hipStream_t s);
 
-// The gathers (pixel shuffle, patches) on the same kernels; p.ws: room for
-// ws_floats floats of split-K partial tiles, or null.
+// The gathers (pixel shuffle, patches) on the same kernels: tile and K splits of
+// a problem with room for ws_floats floats of split-K partial tiles (0: no
+// split; force > 0: that many splits, as far as K and the room allow), the
+// tile's sizes (rows * 1000 + columns), and the launch (p.ws: the room).
+struct GatherPlan {
+  int cfg, splits;
+};
 __attribute__((visibility("hidden"))) bool gather_takes(const GemmArgs& p);
-__attribute__((visibility("hidden"))) int gather_run(const GemmArgs& p, int amode, hipStream_t s,
-                                                     long ws_floats);
+__attribute__((visibility("hidden"))) GatherPlan gather_plan(int M, int N, int K, long ws_floats,
+                                                             int force);
+__attribute__((visibility("hidden"))) int gather_tile(const GatherPlan& g);
+__attribute__((visibility("hidden"))) int gather_run(const GemmArgs& p, int amode,
+                                                     const GatherPlan& g, hipStream_t s);
 
 }  // namespace svla_gemm

@@ -615,23 +615,29 @@ bool gather_takes(const GemmArgs& p) {
 // images 103 / 60, 32 images 133 / 89 (unsplit; 32 and 64 split, but these
 // never shared the workspace), 96 images 225 / 144; patch embedding of 1 image
 // 12.3 / 8.7, 7 images 26.7 / 16.6, 96 images 245 / 174.
-int gather_run(const GemmArgs& p, int amode, hipStream_t s, long ws_floats) {
-  const GatherCfg* best = nullptr;
-  int splits = 1;
-  double best_us = 0;
-  const int nk = (p.K + GK - 1) / GK;
-  for (const GatherCfg& c : kGather)
-    for (int z = 1; z <= kMaxSplits && z * 4 <= nk; ++z) {
-      if (z > 1 && (!p.ws || (long)z * p.M * p.N > ws_floats)) break;
-      const double us = stream_cost(c, p.M, p.N, p.K, z) + split_cost(p.M, p.N, z);
-      if (!best || us < best_us) {
-        best = &c;
+GatherPlan gather_plan(int M, int N, int K, long ws_floats, int force) {
+  const int nk = (K + GK - 1) / GK;
+  if (force <= 0 && nk < 4) return {0, 1};
+  int lo = 1, hi = force > 0 ? min(force, nk) : min(kMaxSplits, nk / 4);
+  hi = (int)max(min((long)hi, ws_floats / ((long)M * N)), 1L);
+  if (force > 0) lo = hi;
+  GatherPlan best{0, 1};
+  double best_us = -1;
+  for (int i = 0; i < (int)(sizeof(kGather) / sizeof(kGather[0])); ++i)
+    for (int z = lo; z <= hi; ++z) {
+      const double us = stream_cost(kGather[i], M, N, K, z) + split_cost(M, N, z);
+      if (best_us < 0 || us < best_us) {
+        best = {i, z};
         best_us = us;
-        splits = z;
       }
     }
-  if (!best) return kGather[0].run(p, amode, 1, s);
-  return best->run(p, amode, splits, s);
+  return best;
+}
+
+int gather_tile(const GatherPlan& g) { return kGather[g.cfg].bm * 1000 + kGather[g.cfg].bn; }
+
+int gather_run(const GemmArgs& p, int amode, const GatherPlan& g, hipStream_t s) {
+  return kGather[g.cfg].run(p, amode, g.splits, s);
 }
 
 int stream_run(const GemmArgs& p, int epi, int act, hipStream_t s) {

@@ -181,8 +181,9 @@ class Group:
 
 # entry points that set state rather than launch work: not timed
 _SKIP = {"svla_init", "svla_version", "svla_gemm_set_tile", "svla_gemm_set_split",
-         "svla_gemm_tile_choice", "svla_gemm_stream_choice", "svla_expert_workspace_size", "svla_expert_prepare",
-         "svla_expert_status", "svla_time_embedding_bf16", "svla_rope_table"}
+         "svla_gemm_tile_choice", "svla_gemm_stream_choice", "svla_gemm_gather_choice",
+         "svla_expert_workspace_size", "svla_expert_prepare", "svla_expert_status",
+         "svla_time_embedding_bf16", "svla_rope_table"}
 
 
 def record_chunk(eng):
