@@ -166,7 +166,9 @@ def test_connector(n, grid, hidden, scale, n_out):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,chans,image,patch,embed", [
     (1, 3, 512, 16, 768), (2, 3, 512, 16, 768), (7, 3, 512, 16, 768), (3, 1, 72, 8, 72),
-    (2, 3, 120, 24, 200)])
+    (2, 3, 120, 24, 200),
+    # short K: every tile that such a gather chooses, ragged rows and columns
+    (1, 3, 512, 8, 776), (5, 3, 520, 8, 776), (24, 1, 224, 8, 200), (52, 1, 224, 8, 392)])
 @pytest.mark.parametrize("pos", [True, False])
 def test_patch_embed(n, chans, image, patch, embed, pos):
     from smolvla import ops
@@ -233,6 +235,20 @@ def test_forced_gather_splits_end_at_k_and_at_the_workspace(force_split):
     # 2^22 floats of partial tiles: 22 times 192 x 960
     assert choice(192, 960, 12288) // 1000000 == 22
     assert choice(320, 960, 12288) // 1000000 == 1        # more rows never split
+
+
+@pytest.mark.parametrize("m,n,k,tile", [
+    (2048, 960, 128, 64064),         # 480 64x64 tiles
+    (4096, 768, 192, 128192),        # 768: one 512-pixel image in 8-pixel patches
+    (49152, 768, 192, 128192), (196608, 768, 192, 256128), (196608, 768, 64, 256128),
+    (18816, 200, 64, 192128), (9408, 384, 192, 128192), (4704, 200, 64, 64064),
+    (4096, 768, 256, 64096),         # four stages: the cost model alone
+])
+def test_gathers_of_short_k(m, n, k, tile):
+    """Under four K stages no more than two 64x64 tiles per CU: past that their
+    fixed costs add up (12 images of 8-pixel patches 76 us, 52 on 128x192)."""
+    from smolvla import _lib
+    assert _lib.load().svla_gemm_gather_choice(m, n, k) == 1000000 + tile
 
 
 def test_dense_skinny_problems_obey_a_forced_split(force_split):

@@ -615,15 +615,25 @@ bool gather_takes(const GemmArgs& p) {
 // images 103 / 60, 32 images 133 / 89 (unsplit; 32 and 64 split, but these
 // never shared the workspace), 96 images 225 / 144; patch embedding of 1 image
 // 12.3 / 8.7, 7 images 26.7 / 16.6, 96 images 245 / 174.
+// Under four K stages a tile is mostly its fixed cost, which the fits (K from
+// 320) do not hold apart: 64x64 tiles up to two per CU, past that the choice
+// among those of 128 rows and more.  MI355X, graph replay, register-staged
+// 128x128 / 64x64 at every size / now: 8-pixel patches of 3 channels (K = 192,
+// N = 768), 1 image 12.0 / 10.1 / 9.1 us, 12 images 65.4 / 76.3 / 52.0, 48
+// images 263 / 311 / 193; K = 64, N = 200, 48 images of 784 patches 17.1 / 19.1
+// / 14.2; a pixel shuffle of 2048x960x128 (480 tiles) 7.1 / 6.0 / 6.0 (128x192
+// 7.2), of 16384x960x128 20.7 / 26.1 / 17.0.
 GatherPlan gather_plan(int M, int N, int K, long ws_floats, int force) {
   const int nk = (K + GK - 1) / GK;
-  if (force <= 0 && nk < 4) return {0, 1};
-  int lo = 1, hi = force > 0 ? min(force, nk) : min(kMaxSplits, nk / 4);
+  const bool brief = nk < 4;
+  if (force <= 0 && brief && (long)((M + 63) / 64) * ((N + 63) / 64) <= 512) return {0, 1};
+  int lo = 1, hi = force > 0 ? min(force, nk) : min(kMaxSplits, max(nk / 4, 1));
   hi = (int)max(min((long)hi, ws_floats / ((long)M * N)), 1L);
   if (force > 0) lo = hi;
   GatherPlan best{0, 1};
   double best_us = -1;
-  for (int i = 0; i < (int)(sizeof(kGather) / sizeof(kGather[0])); ++i)
+  for (int i = 0; i < (int)(sizeof(kGather) / sizeof(kGather[0])); ++i) {
+    if (force <= 0 && brief && kGather[i].bm < 128) continue;
     for (int z = lo; z <= hi; ++z) {
       const double us = stream_cost(kGather[i], M, N, K, z) + split_cost(M, N, z);
       if (best_us < 0 || us < best_us) {
@@ -631,6 +641,7 @@ GatherPlan gather_plan(int M, int N, int K, long ws_floats, int force) {
         best_us = us;
       }
     }
+  }
   return best;
 }
 
