@@ -228,9 +228,9 @@ int svla_gemm_tile_choice(int m, int n, int k, int act);
 
 /* Query: the block tile (rows * 1000 + columns) of the K-split line-DMA kernel
  * (csrc/gemm_stream.hip) that an automatic call with dense, well aligned
- * operands and no fused norm runs on -- plain epilogue, or `paired` (RoPE /
- * SiLU) -- or 0 where it runs on the configuration svla_gemm_tile_choice
- * names.  These kernels are not among the forceable configurations. */
+ * operands (rows on 128-byte lines) and no fused norm runs on -- plain
+ * epilogue, or `paired` (RoPE / SiLU) -- or 0 where it runs on the
+ * configuration svla_gemm_tile_choice names.  These kernels are not among the forceable configurations. */
 int svla_gemm_stream_choice(int m, int n, int k, int paired);
 
 /* Query: K splits * 1000000 + block tile (rows * 1000 + columns) with which a

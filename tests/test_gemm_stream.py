@@ -296,3 +296,32 @@ def test_paired_at_forced_splits(force_split, m, n, k):
     for z in (-1, 1, 2, 4):
         force_split(z)
         _close(ops.linear_silu_mul(a.cuda(), W), (s * up).to(BF16), gate * up, up * s)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,skinny", [
+    (65, 1600, 720, True), (128, 960, 720, True), (100, 2048, 264, True), (65, 960, 1480, True),
+    (100, 2112, 720, False), (100, 960, 200, False), (100, 960, 1544, False)])
+def test_paired_rows_off_lines_keep_the_skinny_tile(m, n, k, skinny):
+    """Packed rows (65 to 128 of them) that do not all start on 128-byte lines
+    give the bits of the 16-column skinny tile, past its range those of rows on
+    lines, which run on the K-split tile."""
+    from smolvla import _lib, ops
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(BF16).cuda()
+    lined = torch.empty(m, (k + 63) // 64 * 64, dtype=BF16, device="cuda")[:, :k].copy_(a)
+    w = ops.pack_weight((torch.randn(k, n, generator=g) * 0.05).to(BF16).cuda())
+    cos_t, sin_t = ops.rope_table(m, 64, 1e5)
+
+    def run(x):
+        lo = torch.zeros(m, n, dtype=BF16, device="cuda")
+        return torch.stack([ops.linear_rope(x, w, n, m, cos_t, sin_t, out_lo=lo), lo])
+
+    got = run(a)
+    assert lib.svla_gemm_set_tile(12 if skinny else -1) == 0
+    try:
+        want = run(a if skinny else lined)
+    finally:
+        lib.svla_gemm_set_tile(-1)
+    assert torch.equal(got, want)

@@ -52,7 +52,7 @@ def test_views_and_inputs_kept():
     _same(lambda x: vision_block(x, pv), x_of(12, 1024, 768))   # every projection slab-blocked
 
 
-@pytest.mark.parametrize("L", [64, 65, 100])
+@pytest.mark.parametrize("L", [64, 65, 100, 128, 129, 300])
 def test_rows_on_lines(L):
     """Weights and norm outputs whose rows start on 128-byte lines give the
     bits of packed ones (below and from LINE_MIN_ROWS)."""

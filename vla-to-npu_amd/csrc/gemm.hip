@@ -2316,14 +2316,19 @@ int pick_split(int tiles, int K, int bm, int bn) {
 // 5.9 / 7.2, down 439x960x2560 10.9 / 12.8; RoPE / SiLU within one 32x64 tile
 // per CU -- 241x1600x960 6.2 / 7.7, 400x960x720 6.1 / 7.0, but 330x1600x720
 // (275 tiles) 7.8 / 7.0 and 400x1600x720 (325) 7.9 / 7.2; up to 64 rows the
-// 16-column skinny tile -- 50x960x720 5.1 / 6.3, 50x4096x720 5.6 / 6.1, but
-// 128x1600x960 8.3 / 7.6 and 128x5120x960 9.6 / 6.9.
-bool small_range(int M, int N, int K, int epi) {
+// 16-column skinny tile -- 50x960x720 5.1 / 6.3, 50x4096x720 5.6 / 6.1.  From 65
+// to 128 rows it depends on where the activation rows start: the skinny tile
+// reads them in 64-byte pieces, faster when they do not all start on a 128-byte
+// line -- rows of 1440 bytes, 100x1600x720 6.0 / 7.0, 128x960x720 5.9 / 6.9, K =
+// 264 to 1480 alike; rows of 1536 bytes, 100x1600x720 7.1 / 7.0; 128x1600x960
+// (1920) 8.6 / 7.6.  Below K = 256 both are within 0.3 us; from 1536 the skinny
+// tile would split K, on the workspace that no further call shall need.
+bool small_range(int M, int N, int K, int epi, long lda) {
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   const bool paired = epi == EPI_ROPE || epi == EPI_SILU;
   if (M > 512 || K < LBK) return K < LBK;
   if (!paired) return tiles(32, 32) <= 2 * kNumCU;
-  if (M <= 64) return tiles(64, 16) <= kNumCU;
+  if (M <= 64 || (M <= 128 && lda % 64 && K >= 256 && K < 1536)) return tiles(64, 16) <= kNumCU;
   return M > 128 && tiles(32, 64) <= kNumCU;
 }
 
@@ -2332,9 +2337,9 @@ bool skinny_tile(TileId t) { return t == S32 || t == S64 || t == S16; }
 // The K-split line-DMA kernels take the mid-size dense problems: everything but
 // the small tiles' and the 256x256 kernel's own ranges, and skinny problems
 // whose K splits are forced (svla_gemm_set_split).
-bool stream_range(int M, int N, int K, int epi, TileId t) {
+bool stream_range(int M, int N, int K, int epi, long lda, TileId t) {
   return g_force_tile < 0 && t != W256 && !(g_force_split > 1 && skinny_tile(t)) &&
-         !small_range(M, N, K, epi);
+         !small_range(M, N, K, epi, lda);
 }
 
 // Whether a gather may split K: only where the skinny tiles' choice is a split
@@ -2393,7 +2398,7 @@ int run_gemm(GemmArgs& p, int epi, int act, hipStream_t s, WsKind wk = WS_ALLOCA
   const bool wide_rows_ok = !p.out_f32 && p.N % 8 == 0 && p.ldc % 8 == 0 &&
                             (!p.res || (p.ldr % 8 == 0 && svla_aligned16(p.res)));
   const TileCfg t = pick_tile(p.M, p.N, p.K, epi, plain, wide_rows_ok, AMODE == A_DENSE);
-  if (AMODE == A_DENSE && stream_range(p.M, p.N, p.K, epi, t.id) && stream_takes(p, epi))
+  if (AMODE == A_DENSE && stream_range(p.M, p.N, p.K, epi, p.lda, t.id) && stream_takes(p, epi))
     return stream_run(p, epi, act, s);
   if (AMODE != A_DENSE && g_force_tile < 0 && epi == EPI_STORE && gather_takes(p)) {
     // (a capture that comes before the workspace exists runs unsplit)
@@ -2485,8 +2490,8 @@ int svla_gemm_tile_choice(int m, int n, int k, int act) {
 
 int svla_gemm_stream_choice(int m, int n, int k, int paired) {
   if (m <= 0 || n <= 0 || n % (paired ? 64 : 8) || k < 8 || k % 8) return SVLA_EINVAL;
-  const int epi = paired ? EPI_ROPE : EPI_STORE;
-  if (!stream_range(m, n, k, epi, pick_tile(m, n, k, epi, !paired, true, true).id)) return 0;
+  const int epi = paired ? EPI_ROPE : EPI_STORE, lda = (k + 63) / 64 * 64;
+  if (!stream_range(m, n, k, epi, lda, pick_tile(m, n, k, epi, !paired, true, true).id)) return 0;
   return stream_tile(m, n, k, epi);
 }
 
@@ -2536,7 +2541,7 @@ int svla_linear_pair_bf16(const void* a0, const void* a1, int lda, const void* w
   // still within the two workgroups per CU up to which the small tile is
   // chosen for one product (MI355X, graph replay, the cross layer around
   // 241x320x320 twice, 80 tiles each: 55.0 us in two launches, 51.4 in one).
-  if (ok && g_force_tile < 0 && small_range(m, n, k, EPI_STORE) &&
+  if (ok && g_force_tile < 0 && small_range(m, n, k, EPI_STORE, lda) &&
       pick_tile(m, n, k, EPI_STORE, true, n % 8 == 0 && ldc % 8 == 0, true).id == N32 &&
       (long)((m + 31) / 32) * ((n + 31) / 32) <= kNumCU) {
     p.a2 = q.a;

@@ -79,8 +79,9 @@ def _pack_cols(ws, device):
 # row that starts on a 128-byte line is one line, of others (K = 720: 1440-byte
 # rows) two.  MI355X, graph replay, rows as packed / on lines: batch-32 chunk
 # 38.54 / 38.02 ms; norm outputs alone, expert self layer 32x50 74.3 / 73.2 us.
-# Up to 64 rows packed ones stay: the skinny tiles are faster on them.
-LINE_MIN_ROWS = 65
+# Up to 128 rows packed ones stay: Q and QKV then run on the skinny tile, which
+# is faster on them (100 rows: Q + RoPE 5.7 / 6.8 us, QKV + RoPE 6.0 / 7.0).
+LINE_MIN_ROWS = 129
 
 
 def _line_empty(rows, cols, device):
