@@ -958,12 +958,17 @@ __global__ __launch_bounds__(256, 2) void gemm_line_kernel(GemmArgs p) {
 // fragment rounded as bf16((x * r) * w) on the way into the MFMAs).
 constexpr int SNS = 4;  // ring stages
 
-template <int BM, int BN, int AMODE, bool NORM, int EPI, int ACT>
+// PAIR: blockIdx.z picks the first or the second product.  A kernel of its own:
+// with the choice in every small tile a call lost 0.05 to 0.25 us (down
+// 50x960x2560 7.7 / 7.9 us, O 50x720x960 5.13 / 5.20).
+template <int BM, int BN, int AMODE, bool NORM, int EPI, int ACT, bool PAIR = false>
 __global__ __launch_bounds__(256, (BM * BN <= 2048 ? 2 : 1)) void gemm_small_kernel(GemmArgs p) {
-  if (gridDim.z > 1 && blockIdx.z) {  // uniform
-    p.a = p.a2;
-    p.b = p.b2;
-    p.c = p.c2;
+  if constexpr (PAIR) {
+    if (blockIdx.z) {  // uniform
+      p.a = p.a2;
+      p.b = p.b2;
+      p.c = p.c2;
+    }
   }
   constexpr int TM = BM / 32;          // 16-row MFMA tiles per wave
   constexpr int TN = BN / 16;          // 16-column MFMA tiles per wave
@@ -2547,8 +2552,10 @@ int svla_linear_pair_bf16(const void* a0, const void* a1, int lda, const void* w
     p.a2 = q.a;
     p.b2 = q.b;
     p.c2 = q.c;
-    return dispatch<A_DENSE, false>(p, EPI_STORE, 0, N32, dim3((n + 31) / 32, (m + 31) / 32, 2),
-                                    (hipStream_t)stream);
+    hipLaunchKernelGGL((gemm_small_kernel<32, 32, A_DENSE, false, EPI_STORE, 0, true>),
+                       dim3((n + 31) / 32, (m + 31) / 32, 2), dim3(256), 0, (hipStream_t)stream, p);
+    SVLA_CHECK_LAUNCH();
+    return SVLA_OK;
   }
   const int rc = run_gemm<A_DENSE>(p, EPI_STORE, 0, (hipStream_t)stream);
   return rc ? rc : run_gemm<A_DENSE>(q, EPI_STORE, 0, (hipStream_t)stream);
