@@ -75,3 +75,19 @@ def test_rows_on_lines(L):
         layers.cross_layer(z, ck, cv, C, cfg, 1, L, 70, rope)
         got.append((y, kv, z))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("rows", [1, 37])
+def test_exported_kv_are_tensors_of_their_own(rows):
+    """K and V share no storage and no version: keeping one does not hold the
+    other, an edit of one is none of the other."""
+    from smolvla.config import DecoderConfig
+    from smolvla.vla.text_encoder_bf16 import text_encoder_forward
+    p = decoder_layer_params(_Gen(7, device="cuda", norm_init="random"), DecoderConfig())
+    x = torch.randn(rows, 960, device="cuda").to(BF16)
+    _, key, value = text_encoder_forward(x, p)
+    for t in (key, value):
+        assert t.is_contiguous() and t.untyped_storage().nbytes() == t.numel() * 2
+    kept = value._version
+    key.zero_()
+    assert value._version == kept and value.any()

@@ -45,8 +45,8 @@ def text_encoder_forward(x_np, params, cfg: DecoderConfig = DEFAULT_CFG, mask="c
     mid = torch.empty_like(out) if kv_export == "torch_ref" else None
     qkv = layers.decoder_layer(x2, P, cfg, B, L, rope, mask, prefix_len, bufs, mid_out=mid, out=out)
     if kv_export == "cache":
-        # K and V leave the fused projection in one copy
-        key, value = qkv[:, qd:].view(B * L, 2, kvd).transpose(0, 1).contiguous().unbind(0)
+        # (two copies: a caller that keeps, saves or edits one holds only that one)
+        key, value = qkv[:, qd:qd + kvd].clone(), qkv[:, qd + kvd:].clone()
     elif kv_export == "torch_ref":
         hn = ops.rmsnorm(mid, P["n1"], resolve_eps(cfg.rms_eps))
         key = ops.linear(hn, P["wqkv"][qd:qd + kvd])
