@@ -23,6 +23,8 @@ pytestmark = pytest.mark.gpu
     (144, 1600, 33, 1),     # three row tiles: 2x2 with an empty fourth
     (144, 1600, 17, 1),     # two row tiles, one row in the second: 1x2
     (144, 1600, 25, 2),     # two samples: QKV keeps one row group
+    (1280, 192, 50, 1),     # 80 column tiles: O and down 1x2 with the plain epilogue
+    (2048, 192, 64, 1),     # the same with 128 column tiles, every row in use
 ])
 def test_unit_forms(hidden, inter, chunk, batch):
     from smolvla.pipeline import SmolVLAEngine

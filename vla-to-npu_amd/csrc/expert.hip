@@ -13,8 +13,9 @@
 //
 // Design (CDNA4; the figures are MI355X measurements of this build):
 //  * One workgroup of 8 waves per CU.  A phase is split into UNITS (an
-//    output tile of a GEMM: the whole rows x 16 columns, or 32 x 32 for paired
-//    projections; one (sample, head) of an attention); unit u of a phase runs on team rank u % team_size.
+//    output tile of a GEMM: 64, 32 or 16 rows x 16 columns, or 32 or 16 rows x
+//    32 columns where that halves the rows a unit reads; one (sample, head) of
+//    an attention); unit u of a phase runs on team rank u % team_size.
 //  * Phases hand over through device-scope arrival counters: a workgroup
 //    that finished its units of phase p waits for its stores to be
 //    acknowledged (vmcnt = 0), then adds its unit count to one of 16
@@ -152,7 +153,7 @@ typedef const __attribute__((address_space(4))) XPhase CPhase;
 struct XArgs {
   CPhase* ph;
   int n_ph;
-  unsigned* cnt;     // [n_ph + 1][kSub][kCntStride]; the last row is the team registration
+  unsigned* cnt;     // [n_ph + 1][kRep][kSub][kCntStride]; the last row is the team registration
   unsigned* status;  // XStat of the launch (0 = ok)
   int team_xcd;      // < 0: every workgroup; else the workgroups on this XCD
   int team_size;     // participants expected when team_xcd >= 0
