@@ -2081,6 +2081,19 @@ TileCfg pick_tile(int M, int N, int K, int epi, bool plain, bool wide_rows_ok, b
     if (g_force_tile == N96 && paired) return tile_dims(N32x64);
     return tile_dims((TileId)g_force_tile);
   }
+  // What reaches the rules below.  Automatic dense bf16 calls without a fused
+  // norm, with N and the leading dimensions multiples of 8, run on
+  // gemm_stream.hip where stream_range says so; of these rules they take the
+  // small tiles, the 16-column skinny tile and the 256x256 kernel.  The rest
+  // serves fp32 outputs, N % 8 != 0, fused norms, the Euler and row-remapped
+  // epilogues, K < 64 and the gathers that gather_takes refuses.  The figures
+  // compare these tiles with each other.
+  // 96 x 96 small tiles for long-K problems of at most one such tile per CU,
+  // measured on MI355X with graph replay: 3072x768x3072 (256 tiles; 64x64 line
+  // tile, 576 tiles) 31.7 -> 27.4 us; short K loses (3072x768x768: 12.1 -> 13.5,
+  // 3072x2304x768 19.1 -> 32.1)
+  if (dense && !paired && K >= 2048 && M >= 2048 && tiles(96, 96) <= kNumCU)
+    return tile_dims(N96);
   // 32-row small tiles (gemm_small_kernel) for dense problems up to 512 rows
   // while the grid stays within two workgroups per CU, measured on MI355X with
   // graph replay: the batch-1 prefix (241 rows) down 241x960x2560 14.1 ->
@@ -2091,15 +2104,7 @@ TileCfg pick_tile(int M, int N, int K, int epi, bool plain, bool wide_rows_ok, b
   // 8.5 -> 6.3.  Not for paired epilogues up to 128 rows (norm + QKV + RoPE
   // 50x1600x720: 6.2 us on the 16-column skinny tile, 6.5 here), nor past 512
   // tiles (norm + gate|up 241x5120x960: 12.0 on the 64x64 line tile, 13.2
-  // here; expert O 1600x720x960: 9.9 vs 10.5), nor for the gathers (connector
-  // 192x960x12288: 40.2 vs 47.7, patch embedding 18.8 vs 23.3).
-  // 96 x 96 small tiles for long-K problems of one such tile per CU, measured
-  // on MI355X with graph replay: the batch-1 ViT down projection 3072x768x3072
-  // 31.7 -> 27.4 us (256 tiles; its 64x64 line tile runs 576); short K loses
-  // (ViT O 3072x768x768: 12.1 -> 13.5, QKV 19.1 -> 32.1), and so do the
-  // paired / 64-column variants on every engine shape measured
-  if (dense && !paired && K >= 2048 && M >= 2048 && tiles(96, 96) <= kNumCU)
-    return tile_dims(N96);
+  // here).
   if (dense && M <= 512 && K >= LBK) {
     if (!paired && tiles(32, 32) <= 2 * kNumCU) return tile_dims(N32);
     if (paired && M > 128 && tiles(32, 64) <= 2 * kNumCU) return tile_dims(N32x64);
@@ -2138,58 +2143,46 @@ TileCfg pick_tile(int M, int N, int K, int epi, bool plain, bool wide_rows_ok, b
   // 752 us; K = 3072: 1603 vs 2285 us) and loses below (K = 256: 465 vs 430)
   if (wide_ok && K >= 512 && tiles(WBM, WBN) >= 2 * kNumCU) return tile_dims(W256);
   const bool line_ok = K >= LBK;
-  // dense A from M = 4096 (the batch-32 prefix, 7712 rows; its RMSNorm runs
-  // on its own there), measured on MI355X with graph replay: the 128x128
-  // line-DMA tile beats the register-staged 128x128 kernel and the other
-  // pipelines on every prefix GEMM -- down 7712x960x2560 47.2 us, O
-  // 7712x960x960 25.3, QKV + RoPE 7712x1600x960 43.8 (46.7 on 64x128), gate|up
-  // + SiLU 7712x5120x960 93.4 (116.4 register-staged); a grid under one
-  // 128x128 tile per CU takes the 64x64 line tile (the cross K/V projection
-  // 7712x320x320: 9.4 -> 7.6 us).
-  // (gathers reach this choice only with outputs that the gather kernels of
-  // gemm_stream.hip do not take)
+  // from M = 4096, measured on MI355X with graph replay: the 128x128 line-DMA
+  // tile beats the register-staged 128x128 kernel and the other pipelines --
+  // 7712x5120x960 + SiLU 93.4 us (116.4 register-staged), 7712x1600x960 + RoPE
+  // 43.8 (46.7 on 64x128); a grid under one 128x128 tile per CU takes the 64x64
+  // line tile (7712x320x320: 9.4 -> 7.6 us)
   if (!dense && M >= 4096) return tile_dims(T128);
   if (dense && M >= 4096) {
     if (!line_ok) return tile_dims(T128);
     if (tiles(128, 128) < kNumCU) return tile_dims(L64);
     return tile_dims(L128);
   }
-  // from M = 3072 (the batch-1 ViT, 3 images), measured on MI355X, line-DMA
-  // tiles: up 3072x3072x768 + GELU 38.0 -> 27.8 us (128x64), QKV
-  // 3072x2304x768 22.9 -> 18.8 (128x128), down 3072x768x3072 35.8 -> 29.9 and
-  // O 3072x768x768 14.0 -> 11.2 (64x64)
+  // from M = 3072, measured on MI355X, line-DMA tiles: 3072x3072x768 + GELU
+  // 38.0 -> 27.8 us (128x64), 3072x2304x768 22.9 -> 18.8 (128x128),
+  // 3072x768x3072 35.8 -> 29.9 and 3072x768x768 14.0 -> 11.2 (64x64)
   if (M >= 3072 && line_ok && !paired) {
     if (N >= 3072) return tile_dims(L128x64);
     if (N >= 2048) return tile_dims(L128);
     return tile_dims(L64);
   }
-  // from M = 3072 (the batch-1 ViT, 3 images) too, measured on MI355X: up
-  // 3072x3072x768 + GELU 38.1 -> 35.0 us, down 3072x768x3072 42.7 -> 34.1 us,
-  // QKV and O within 0.4 us
+  // from M = 3072 too (K < 64, paired), measured on MI355X: 3072x3072x768 + GELU
+  // 38.1 -> 35.0 us, 3072x768x3072 42.7 -> 34.1
   if (M >= 3072 || tiles(128, 128) >= 4 * kNumCU) return pipe_ok ? tile_dims(P128) : tile_dims(T128);
-  // mid-size (the batched expert, M = 1600), measured on MI355X: with at least
+  // mid-size, measured on MI355X: with at least
   // one 128x128 tile per CU the 32x32-MFMA register-staged 128x128 kernel wins
   // (gate|up 1600x4096x720: 19 us vs 34 us on 64x64); below that the 64x64
   // LDS-DMA pipeline's larger grid wins
   if (tiles(128, 128) >= kNumCU) return tile_dims(T128);
   if (!pipe_ok) return tile_dims(T64);
-  // paired epilogues below one 128x128 tile per CU, measured on MI355X (the
-  // expert at batch 32, M = 1600): the 64x64 line-DMA tile -- norm + QKV +
-  // RoPE 1600x1600x720 19.3 -> 14.5 us, norm + Q + RoPE 1600x960x720 12.2 ->
-  // 11.1
+  // paired epilogues below one 128x128 tile per CU, measured on MI355X: the
+  // 64x64 line-DMA tile -- norm + QKV + RoPE 1600x1600x720 19.3 -> 14.5 us,
+  // norm + Q + RoPE 1600x960x720 12.2 -> 11.1
   if (paired && line_ok) return tile_dims(L64);
   // below that, measured on MI355X: when the 64x64 grid would put one or two
   // workgroups on each CU (256-512 tiles, uneven), a 128x64 / 64x128 tile
-  // halves the grid to about one per CU (expert at batch 32, M = 1600: O
-  // 12.5 -> 10.9 us, down 19.3 -> 16.9 us, Q + RoPE 12.1 -> 11.0 us; M =
-  // 1928, K = 2560: 25.4 -> 22.4 us); with fewer tiles, or more (the batch-1
-  // ViT's 576), 64x64 stays ahead.  Paired epilogues need 64-wide wave tiles:
-  // 64x128, or 128x128 for large paired grids (QKV + RoPE 1600 x 720:
-  // 17.7 -> 15.2 us).
-  // Re-measured with the current kernels (graph replay, M = 1600): the
-  // 128x64 tile still wins for long K (down, K = 2048: 17.8 vs 19.9 us) but
-  // not for short K (time MLP 1600x720x720: 10.3 vs 9.4 us on 64x64; O,
-  // K = 960: 11.0 vs 10.6).
+  // halves the grid to about one per CU (M = 1928, K = 2560: 25.4 -> 22.4 us);
+  // with fewer tiles, or more (576), 64x64 stays ahead.  Paired epilogues need
+  // 64-wide wave tiles: 64x128, or 128x128 for large paired grids (QKV + RoPE
+  // 1600 x 720: 17.7 -> 15.2 us).  At M = 1600 the 128x64 tile wins for long K
+  // (K = 2048: 17.8 vs 19.9 us) but not for short K (1600x720x720: 10.3 vs 9.4
+  // us on 64x64; K = 960: 11.0 vs 10.6).
   const long t64 = tiles(64, 64);
   if (t64 >= kNumCU && t64 <= 2 * kNumCU && (paired || K > 1024))
     return tile_dims(paired ? P64x128 : P128x64);
