@@ -301,7 +301,8 @@ def test_paired_at_forced_splits(force_split, m, n, k):
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,skinny", [
     (65, 1600, 720, True), (128, 960, 720, True), (100, 2048, 264, True), (65, 960, 1480, True),
-    (100, 2112, 720, False), (100, 960, 200, False), (100, 960, 1544, False)])
+    (100, 2112, 720, False), (100, 960, 200, True), (128, 1536, 72, True),
+    (128, 2048, 200, False), (100, 960, 1544, False)])
 def test_paired_rows_off_lines_keep_the_skinny_tile(m, n, k, skinny):
     """Packed rows (65 to 128 of them) that do not all start on 128-byte lines
     give the bits of the 16-column skinny tile, past its range those of rows on

@@ -2319,14 +2319,18 @@ int pick_split(int tiles, int K, int bm, int bn) {
 // reads them in 64-byte pieces, faster when they do not all start on a 128-byte
 // line -- rows of 1440 bytes, 100x1600x720 6.0 / 7.0, 128x960x720 5.9 / 6.9, K =
 // 264 to 1480 alike; rows of 1536 bytes, 100x1600x720 7.1 / 7.0; 128x1600x960
-// (1920) 8.6 / 7.6.  Below K = 256 both are within 0.3 us; from 1536 the skinny
-// tile would split K, on the workspace that no further call shall need.
+// (1920) 8.6 / 7.6.  Below K = 256 only RoPE, up to three tiles per four CUs --
+// rows of 400 bytes, 96x704x200 4.2 / 4.6, 128x2048x200 4.8 / 4.7; SiLU is faster
+// on the stream kernels (111x384x200 4.0 / 3.9).  From K = 1536 the skinny tile
+// would split K, on the workspace that no further call shall need.
 bool small_range(int M, int N, int K, int epi, long lda) {
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   const bool paired = epi == EPI_ROPE || epi == EPI_SILU;
   if (M > 512 || K < LBK) return K < LBK;
   if (!paired) return tiles(32, 32) <= 2 * kNumCU;
-  if (M <= 64 || (M <= 128 && lda % 64 && K >= 256 && K < 1536)) return tiles(64, 16) <= kNumCU;
+  if (M <= 64) return tiles(64, 16) <= kNumCU;
+  if (M <= 128 && lda % 64 && K < 256) return epi == EPI_ROPE && tiles(64, 16) <= 3 * kNumCU / 4;
+  if (M <= 128 && lda % 64 && K < 1536) return tiles(64, 16) <= kNumCU;
   return M > 128 && tiles(32, 64) <= kNumCU;
 }
 
