@@ -611,10 +611,11 @@ bool gather_takes(const GemmArgs& p) {
 // K = 12288, so with one its K is split over workgroups as far as `ws_floats`
 // floats hold the partial tiles.  MI355X, graph replay, before (64x64 line
 // tile, register-staged 128x128 or split skinny tiles) / now: connector of 1
-// image 22.0 / 13.9 us, 3 images 40.4 / 21.5, 4 images 42.1 / 23.8 (split), 9
+// image 22.0 / 13.9 us, 3 images 38.4 / 19.4, 4 images 42.1 / 23.8 (split), 9
 // images 103 / 60, 32 images 133 / 89 (unsplit; 32 and 64 split, but these
 // never shared the workspace), 96 images 225 / 144; patch embedding of 1 image
-// 12.3 / 8.7, 7 images 26.7 / 16.6, 96 images 245 / 174.
+// 12.3 / 8.7, 7 images 26.7 / 16.6, 96 images 235 / 171.  The connector's K lies
+// past that of the fits: for 96 images they say 106 us.
 // Under four K stages a tile is mostly its fixed cost, which the fits (K from
 // 320) do not hold apart: 64x64 tiles up to two per CU, past that the choice
 // among those of 128 rows and more.  MI355X, graph replay, register-staged
