@@ -46,7 +46,7 @@ def text_encoder_forward(x_np, params, cfg: DecoderConfig = DEFAULT_CFG, mask="c
     qkv = layers.decoder_layer(x2, P, cfg, B, L, rope, mask, prefix_len, bufs, mid_out=mid, out=out)
     if kv_export == "cache":
         # (two copies: a caller that keeps, saves or edits one holds only that one)
-        key, value = qkv[:, qd:qd + kvd].clone(), qkv[:, qd + kvd:].clone()
+        key, value = torch.split_with_sizes_copy(qkv[:, qd:], (kvd, kvd), 1)
     elif kv_export == "torch_ref":
         hn = ops.rmsnorm(mid, P["n1"], resolve_eps(cfg.rms_eps))
         key = ops.linear(hn, P["wqkv"][qd:qd + kvd])
